@@ -1,0 +1,123 @@
+// gemm_common.h -- element types, MFMA forms, epilogue arithmetic and tile
+// walk shared by the GEMM kernels (gemm_kernels.hip, gemm_tiles.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "../hiplayer.h"
+#include "blasx_ext.h"
+#include "gmem.h"
+
+namespace {
+
+typedef double d4_t __attribute__((ext_vector_type(4)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+
+struct cplx {
+    double re, im;
+};
+
+template <typename E> struct Cfg;
+// OUT_ROW(lg, v): the 16x16 MFMA output row held by accumulator element v
+// of a lane in lane-group lg = lane / 16 (column = lane % 16).  Measured on
+// gfx950: the FP32 16x16x4 MFMA returns rows 4*lg + v, the FP64 16x16x4
+// MFMA returns rows lg + 4*v.
+template <> struct Cfg<double> {
+    static constexpr int BM = 128, BN = 128, BK = 16, VEC = 2, PADA = 2, PADB = 2;
+    typedef d4_t acc_t;
+    static __device__ __forceinline__ int out_row(int lg, int v) { return lg + 4 * v; }
+};
+template <> struct Cfg<float> {
+    static constexpr int BM = 128, BN = 128, BK = 32, VEC = 4, PADA = 4, PADB = 4;
+    typedef f4_t acc_t;
+    static __device__ __forceinline__ int out_row(int lg, int v) { return 4 * lg + v; }
+};
+template <> struct Cfg<cplx> {
+    static constexpr int BM = 128, BN = 64, BK = 8, VEC = 1, PADA = 1, PADB = 1;
+    typedef d4_t acc_t;
+    static __device__ __forceinline__ int out_row(int lg, int v) { return lg + 4 * v; }
+};
+
+constexpr int NT = 256;
+enum { MAJ_MN = 0, MAJ_K = 1 };
+
+template <typename E> __device__ __forceinline__ E zero_of() { return E(0); }
+template <> __device__ __forceinline__ cplx zero_of<cplx>() { return cplx{0.0, 0.0}; }
+
+template <typename E> __device__ __forceinline__ E conj_of(E x) { return x; }
+template <> __device__ __forceinline__ cplx conj_of<cplx>(cplx x) { return cplx{x.re, -x.im}; }
+
+// The epilogue's arithmetic, one rounding sequence for every kernel (explicit
+// FMAs: no result depends on how the compiler contracts a kernel's code).
+// alpha * s, then + beta * c in one FMA; c is not used when beta_zero.
+template <typename E>
+__device__ __forceinline__ E out_real(E alpha, E s, E beta, E c, bool beta_zero)
+{
+    const E x = alpha * s;
+    return beta_zero ? x : fma(beta, c, x);
+}
+// complex: alpha (sr + i sim), then + beta c
+__device__ __forceinline__ cplx out_cplx(double ar, double ai, double sr, double sim, double br,
+                                         double bi, cplx c, bool beta_zero)
+{
+    double orr = fma(ar, sr, -(ai * sim)), oi = fma(ar, sim, ai * sr);
+    if (!beta_zero) {
+        orr = fma(br, c.re, fma(-bi, c.im, orr));
+        oi = fma(br, c.im, fma(bi, c.re, oi));
+    }
+    return cplx{orr, oi};
+}
+
+__device__ __forceinline__ d4_t mfma(double a, double b, d4_t c)
+{
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f4_t mfma(float a, float b, f4_t c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+__host__ __device__ __forceinline__ bool aligned16(const void *p, int64_t ld, int esize)
+{
+    return ((reinterpret_cast<uintptr_t>(p) & 15) == 0) && (((ld * esize) & 15) == 0);
+}
+
+// block tile index -> (tm, tn), walking groups of 8 tile rows so that the
+// blocks resident at one time share A row panels and B column panels
+template <int G = 8>
+__device__ __forceinline__ void tile_coords(int t, int tiles_m, int tiles_n, int &tm, int &tn)
+{
+    const int per_group = G * tiles_n;
+    const int g = t / per_group;
+    const int first = g * G;
+    const int gsz = min(tiles_m - first, G);
+    const int r = t - g * per_group;
+    tm = first + r % gsz;
+    tn = r / gsz;
+}
+
+// segment i of the table, or the by-value segment when there is no table;
+// fields are read through the global address space one by one (selecting
+// between a table pointer and a local would make every access FLAT)
+__device__ __forceinline__ bxh_seg_t seg_at(const bxh_seg_t *segs, const bxh_seg_t &seg0, int i)
+{
+    if (!segs) return seg0;
+    const __attribute__((address_space(1))) bxh_seg_t *g =
+        (const __attribute__((address_space(1))) bxh_seg_t *)(segs + i);
+    bxh_seg_t s;
+    s.A = g->A;
+    s.B = g->B;
+    s.lda = g->lda;
+    s.ldb = g->ldb;
+    s.k = g->k;
+    return s;
+}
+
+// whether a rank-k update writes element (row, col) of its diagonal block
+__device__ __forceinline__ bool tri_keep(int tri, int row, int col)
+{
+    return (!(tri & BX_TRI_LOWER) || row >= col) && (!(tri & BX_TRI_UPPER) || row <= col);
+}
+
+
+} // namespace

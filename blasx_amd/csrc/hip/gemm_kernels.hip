@@ -26,40 +26,9 @@
 
 #include "../hiplayer.h"
 #include "blasx_ext.h"
-#include "gmem.h"
+#include "gemm_common.h"
 
 namespace {
-
-typedef double d4_t __attribute__((ext_vector_type(4)));
-typedef float f4_t __attribute__((ext_vector_type(4)));
-
-struct cplx {
-    double re, im;
-};
-
-template <typename E> struct Cfg;
-// OUT_ROW(lg, v): the 16x16 MFMA output row held by accumulator element v
-// of a lane in lane-group lg = lane / 16 (column = lane % 16).  Measured on
-// gfx950: the FP32 16x16x4 MFMA returns rows 4*lg + v, the FP64 16x16x4
-// MFMA returns rows lg + 4*v.
-template <> struct Cfg<double> {
-    static constexpr int BM = 128, BN = 128, BK = 16, VEC = 2, PADA = 2, PADB = 2;
-    typedef d4_t acc_t;
-    static __device__ __forceinline__ int out_row(int lg, int v) { return lg + 4 * v; }
-};
-template <> struct Cfg<float> {
-    static constexpr int BM = 128, BN = 128, BK = 32, VEC = 4, PADA = 4, PADB = 4;
-    typedef f4_t acc_t;
-    static __device__ __forceinline__ int out_row(int lg, int v) { return 4 * lg + v; }
-};
-template <> struct Cfg<cplx> {
-    static constexpr int BM = 128, BN = 64, BK = 8, VEC = 1, PADA = 1, PADB = 1;
-    typedef d4_t acc_t;
-    static __device__ __forceinline__ int out_row(int lg, int v) { return lg + 4 * v; }
-};
-
-constexpr int NT = 256;
-enum { MAJ_MN = 0, MAJ_K = 1 };
 
 template <typename E, int VEC> struct alignas(16) Vec {
     E e[VEC];
@@ -68,42 +37,6 @@ template <typename E, int VEC> struct alignas(16) Vec {
 template <typename E, int N> struct alignas(sizeof(E) * N) Lv {
     E e[N];
 };
-
-template <typename E> __device__ __forceinline__ E zero_of() { return E(0); }
-template <> __device__ __forceinline__ cplx zero_of<cplx>() { return cplx{0.0, 0.0}; }
-
-template <typename E> __device__ __forceinline__ E conj_of(E x) { return x; }
-template <> __device__ __forceinline__ cplx conj_of<cplx>(cplx x) { return cplx{x.re, -x.im}; }
-
-// The epilogue's arithmetic, one rounding sequence for every kernel (explicit
-// FMAs: no result depends on how the compiler contracts a kernel's code).
-// alpha * s, then + beta * c in one FMA; c is not used when beta_zero.
-template <typename E>
-__device__ __forceinline__ E out_real(E alpha, E s, E beta, E c, bool beta_zero)
-{
-    const E x = alpha * s;
-    return beta_zero ? x : fma(beta, c, x);
-}
-// complex: alpha (sr + i sim), then + beta c
-__device__ __forceinline__ cplx out_cplx(double ar, double ai, double sr, double sim, double br,
-                                         double bi, cplx c, bool beta_zero)
-{
-    double orr = fma(ar, sr, -(ai * sim)), oi = fma(ar, sim, ai * sr);
-    if (!beta_zero) {
-        orr = fma(br, c.re, fma(-bi, c.im, orr));
-        oi = fma(br, c.im, fma(bi, c.re, oi));
-    }
-    return cplx{orr, oi};
-}
-
-__device__ __forceinline__ d4_t mfma(double a, double b, d4_t c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f4_t mfma(float a, float b, f4_t c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 // ---------------------------------------------------------------------------
 // Tile loader: ROWS x BK tile of op(X) (rows = the M or N dimension).
@@ -207,25 +140,6 @@ template <typename E, int VEC, int ROWS, int BK, int PAD, int MAJ, bool CONJ> st
     }
 };
 
-__host__ __device__ __forceinline__ bool aligned16(const void *p, int64_t ld, int esize)
-{
-    return ((reinterpret_cast<uintptr_t>(p) & 15) == 0) && (((ld * esize) & 15) == 0);
-}
-
-// block tile index -> (tm, tn), walking groups of 8 tile rows so that the
-// blocks resident at one time share A row panels and B column panels
-__device__ __forceinline__ void tile_coords(int t, int tiles_m, int tiles_n, int &tm, int &tn)
-{
-    constexpr int G = 8;
-    const int per_group = G * tiles_n;
-    const int g = t / per_group;
-    const int first = g * G;
-    const int gsz = min(tiles_m - first, G);
-    const int r = t - g * per_group;
-    tm = first + r % gsz;
-    tn = r / gsz;
-}
-
 // ---------------------------------------------------------------------------
 // LDS -> MFMA for one staged K tile (real types)
 // ---------------------------------------------------------------------------
@@ -327,32 +241,9 @@ template <typename E> struct Smem {
     static constexpr int ELEMS = Blk<E>::ELEMS;
 };
 
-// segment i of the table, or the by-value segment when there is no table;
-// fields are read through the global address space one by one (selecting
-// between a table pointer and a local would make every access FLAT)
-__device__ __forceinline__ bxh_seg_t seg_at(const bxh_seg_t *segs, const bxh_seg_t &seg0, int i)
-{
-    if (!segs) return seg0;
-    const __attribute__((address_space(1))) bxh_seg_t *g =
-        (const __attribute__((address_space(1))) bxh_seg_t *)(segs + i);
-    bxh_seg_t s;
-    s.A = g->A;
-    s.B = g->B;
-    s.lda = g->lda;
-    s.ldb = g->ldb;
-    s.k = g->k;
-    return s;
-}
-
 // ---------------------------------------------------------------------------
 // One block tile of one problem.
 // ---------------------------------------------------------------------------
-// whether a rank-k update writes element (row, col) of its diagonal block
-__device__ __forceinline__ bool tri_keep(int tri, int row, int col)
-{
-    return (!(tri & BX_TRI_LOWER) || row >= col) && (!(tri & BX_TRI_UPPER) || row <= col);
-}
-
 template <typename E, int MAJA, int MAJB, bool CJA, bool CJB, int WTM = 64, int WTN = 64>
 __device__ __forceinline__ void gemm_block(const bxh_problem_t &P, const bxh_seg_t *segs,
                                            const bxh_seg_t &seg0, int tm, int tn, E *smem)
@@ -501,23 +392,6 @@ __device__ __forceinline__ void gemm_block(const bxh_problem_t &P, const bxh_seg
                 }
             }
     }
-}
-
-// ---------------------------------------------------------------------------
-// Kernels
-// ---------------------------------------------------------------------------
-template <typename E, int MAJA, int MAJB, bool CJA, bool CJB>
-__global__ __launch_bounds__(NT, 2) void k_gemm_plain(bxh_problem_t P, bxh_seg_t S)
-{
-    __shared__ __attribute__((aligned(16))) E smem[Smem<E>::ELEMS];
-    int b = blockIdx.x;
-    const int nb = gridDim.x;
-    // The dispatcher places block b on XCD b % 8.  Renumber so each XCD
-    // works on a contiguous range of tiles (shared panels stay in its L2).
-    if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
-    int tm, tn;
-    tile_coords(b, P.tiles_m, P.tiles_n, tm, tn);
-    gemm_block<E, MAJA, MAJB, CJA, CJB>(P, nullptr, S, tm, tn, smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -898,37 +772,6 @@ __device__ __forceinline__ void dma64_block(const bxh_problem_t &P, const bxh_se
         }
 }
 
-template <int MAJA, int MAJB>
-__global__ __launch_bounds__(NT, 2) void k_dgemm_dma(bxh_problem_t P, bxh_seg_t S)
-{
-    __shared__ __attribute__((aligned(16))) double smem[dma64::SMEM_DOUBLES];
-    int b = blockIdx.x;
-    const int nb = gridDim.x;
-    if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
-    int tm, tn;
-    tile_coords(b, P.tiles_m, P.tiles_n, tm, tn);
-    // the nested K loop for NN only (1% faster at 32768^3); NT and TN ran 7-11%
-    // slower with it and TT no faster, so they keep the segment-walking loop
-    dma64_block<MAJA, MAJB, false, MAJA == MAJ_MN && MAJB == MAJ_K>(P, nullptr, S, tm, tn, smem);
-}
-
-// A ragged DGEMM: any M, N and K, aligned operands (edge tiles clamp their
-// operand rows and mask their stores, K tails take one register-staged step).
-template <int MAJA, int MAJB>
-__global__ __launch_bounds__(NT, 2) void k_dgemm_dma_kt(bxh_problem_t P, bxh_seg_t S)
-{
-    __shared__ __attribute__((aligned(16))) double smem[dma64::SMEM_DOUBLES];
-    // blocks go to the 8 XCDs round-robin (block b on XCD b % 8): give XCD x
-    // the contiguous tile range [x q + min(x, r), ...) of its q or q + 1
-    // blocks (nb = 8 q + r), so its blocks share A and B panels in its L2
-    // for any grid size
-    const int nb = gridDim.x, x = blockIdx.x & 7, q = nb >> 3, r = nb & 7;
-    const int b = x * q + (x < r ? x : r) + (blockIdx.x >> 3);
-    int tm, tn;
-    tile_coords(b, P.tiles_m, P.tiles_n, tm, tn);
-    dma64_block<MAJA, MAJB, false, true, true, true>(P, nullptr, S, tm, tn, smem);
-}
-
 // ---------------------------------------------------------------------------
 // ZGEMM with global -> LDS DMA staging (M a multiple of 128, N of 64, K of 8;
 // complex128 operands are always 16-byte aligned).  Same scheme as the FP64
@@ -981,20 +824,6 @@ __device__ __forceinline__ cplx frag(const cplx *stage, int row, int s, int lg)
 template <int MAJA, int MAJB, bool CJA, bool CJB, bool MASK = false, bool NESTED = true>
 __device__ __forceinline__ void dmaz_block(const bxh_problem_t &P, const bxh_seg_t *segs,
                                            const bxh_seg_t &seg0, int tm, int tn, cplx *smem);
-
-template <int MAJA, int MAJB, bool CJA, bool CJB>
-__global__ __launch_bounds__(NT, 2) void k_zgemm_dma(bxh_problem_t P, bxh_seg_t S)
-{
-    __shared__ __attribute__((aligned(16))) cplx smem[2 * (dmaz::BM + dmaz::BN) * dmaz::BK];
-    int b = blockIdx.x;
-    const int nb = gridDim.x;
-    if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
-    int tm, tn;
-    tile_coords(b, P.tiles_m, P.tiles_n, tm, tn);
-    // the segment-walking K loop: the nested one ran 6% slower on every
-    // transpose at 32768^3
-    dmaz_block<MAJA, MAJB, CJA, CJB, false, false>(P, nullptr, S, tm, tn, smem);
-}
 
 // ---------------------------------------------------------------------------
 // SGEMM with global -> LDS DMA staging (M, N multiples of 128, K of 32,
@@ -1253,20 +1082,6 @@ __device__ __forceinline__ void dmas_block(const bxh_problem_t &P, const bxh_seg
                 gstore(c, out_real(alpha, acc[i][j][v], beta, old, (bool)P.beta_zero));
             }
         }
-}
-
-template <int MAJA, int MAJB>
-__global__ __launch_bounds__(NT, 2) void k_sgemm_dma(bxh_problem_t P, bxh_seg_t S)
-{
-    __shared__ __attribute__((aligned(16))) float smem[2 * 2 * dmas::STAGE];
-    int b = blockIdx.x;
-    const int nb = gridDim.x;
-    if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
-    int tm, tn;
-    tile_coords(b, P.tiles_m, P.tiles_n, tm, tn);
-    // the nested K loop: 3-6% faster than the segment-walking one on every
-    // transpose at 32768^3
-    dmas_block<MAJA, MAJB>(P, nullptr, S, tm, tn, smem);
 }
 
 template <int MAJA, int MAJB, bool CJA, bool CJB, bool MASK, bool NESTED>
@@ -1707,39 +1522,12 @@ int fail(const char *what, hipError_t e)
     return BLASX_EHIP;
 }
 
-template <typename E, int MAJA, int MAJB, bool CJA, bool CJB>
-int launch_plain(const bxh_problem_t &P, const bxh_seg_t &S, hipStream_t st)
-{
-    const int grid = P.tiles_m * P.tiles_n;
-    hipLaunchKernelGGL((k_gemm_plain<E, MAJA, MAJB, CJA, CJB>), dim3(grid), dim3(NT), 0, st, P, S);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : fail("gemm launch", e);
-}
-
-template <int MAJA, int MAJB>
-int launch_dgemm_dma(const bxh_problem_t &P, const bxh_seg_t &S, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_dgemm_dma<MAJA, MAJB>), dim3(P.tiles_m * P.tiles_n), dim3(NT), 0, st, P,
-                       S);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : fail("dgemm dma launch", e);
-}
-
-// the DMA-staged FP64 kernel's conditions: no edge tiles, 16-byte aligned
-// operands and leading dimensions
-bool dgemm_dma_ok(const bxh_problem_t &P, const bxh_seg_t &S)
-{
-    return P.m % 128 == 0 && P.n % 128 == 0 && S.k >= 16 && S.k % 16 == 0 &&
-           aligned16(S.A, S.lda, 8) && aligned16(S.B, S.ldb, 8);
-}
-
-// ---- ragged DGEMM on the DMA-staged kernel ----
-// A problem with edge tiles (M or N not a multiple of 128), any K, or
-// operands whose base or leading dimension is not 16-byte aligned runs as one
-// launch of k_dgemm_dma_kt over all its tiles (edge tiles clamp their operand
-// rows and mask their stores).  A misaligned operand is first copied into an
-// aligned workspace (one HBM pass, leading dimension rounded up to 8 doubles)
-// when the product is large enough to pay for it.
+// ---- misaligned DGEMM operands ----
+// An operand whose base or leading dimension is not 16-byte aligned is moved
+// through registers by the tile kernels (64 TFLOP/s at 3001^3, where aligned
+// operands reach 70).  A product large enough to pay for it copies the
+// operand into an aligned workspace first (one HBM pass, leading dimension
+// rounded up to 8 doubles).
 
 __global__ void k_repack(const double *__restrict__ src, int64_t lds, double *__restrict__ dst,
                          int64_t ldd, int64_t rows, int64_t cols)
@@ -1768,15 +1556,6 @@ struct Workspace {
 Workspace g_rws;
 pthread_mutex_t g_rws_lock = PTHREAD_MUTEX_INITIALIZER;
 
-template <int MAJA, int MAJB>
-int launch_dgemm_kt(const bxh_problem_t &P, const bxh_seg_t &S, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_dgemm_dma_kt<MAJA, MAJB>), dim3(P.tiles_m * P.tiles_n), dim3(NT), 0, st,
-                       P, S);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : fail("dgemm dma (ragged) launch", e);
-}
-
 // rows x cols of the stored operand behind op(A) (m x k) / op(B) (k x n)
 inline void stored_dims(int op, int64_t r, int64_t c, int64_t &rows, int64_t &cols)
 {
@@ -1784,11 +1563,13 @@ inline void stored_dims(int op, int64_t r, int64_t c, int64_t &rows, int64_t &co
     cols = op ? r : c;
 }
 
-// 1: ran; 0: not taken (the caller runs the plain kernel); <0: error
-int dgemm_ragged(int ta, int tb, const bxh_problem_t &P, const bxh_seg_t &S, hipStream_t st)
+// 1: ran; 0: not taken (the caller runs the product on the operands as they
+// are); <0: error
+int dgemm_repacked(int ta, int tb, const bxh_problem_t &P, const bxh_seg_t &S, hipStream_t st)
 {
-    if (P.m < 128 || P.n < 128 || S.k < 16 || P.tri) return 0;
+    if (P.m < 128 || P.n < 128 || S.k < 16) return 0;
     const bool okA = aligned16(S.A, S.lda, 8), okB = aligned16(S.B, S.ldb, 8);
+    if (okA && okB) return 0;
     // a copy of A costs ~16 MK bytes against 2 MNK flops: worth it from N ~ 4096
     if ((!okA && P.n < 4096) || (!okB && P.m < 4096)) return 0;
     int64_t ra, ca, rb, cb;
@@ -1797,133 +1578,39 @@ int dgemm_ragged(int ta, int tb, const bxh_problem_t &P, const bxh_seg_t &S, hip
     const int64_t lda2 = (ra + 7) & ~(int64_t)7, ldb2 = (rb + 7) & ~(int64_t)7;
     const size_t bytesA = okA ? 0 : (size_t)lda2 * ca * 8, bytesB = okB ? 0 : (size_t)ldb2 * cb * 8;
     bxh_seg_t S2 = S;
-    const bool ws = bytesA + bytesB > 0;
-    if (ws) {
-        pthread_mutex_lock(&g_rws_lock);
-        hipError_t e = hipSuccess;
-        if (!g_rws.done) e = hipEventCreateWithFlags(&g_rws.done, hipEventDisableTiming);
-        if (e == hipSuccess && bytesA + bytesB > g_rws.cap) {
-            e = hipEventSynchronize(g_rws.done);
-            if (e == hipSuccess && g_rws.p) e = hipFree(g_rws.p);
-            g_rws.p = nullptr;
-            g_rws.cap = 0;
-            if (e == hipSuccess) e = hipMalloc(&g_rws.p, bytesA + bytesB);
-            if (e == hipSuccess) g_rws.cap = bytesA + bytesB;
-        }
-        if (e == hipSuccess) e = hipStreamWaitEvent(st, g_rws.done, 0);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            pthread_mutex_unlock(&g_rws_lock);
-            return fail("ragged dgemm workspace", e);
-        }
-        double *wa = (double *)g_rws.p, *wb = (double *)((char *)g_rws.p + bytesA);
-        if (!okA) {
-            launch_repack((const double *)S.A, S.lda, wa, lda2, ra, ca, st);
-            S2.A = wa;
-            S2.lda = lda2;
-        }
-        if (!okB) {
-            launch_repack((const double *)S.B, S.ldb, wb, ldb2, rb, cb, st);
-            S2.B = wb;
-            S2.ldb = ldb2;
-        }
+    pthread_mutex_lock(&g_rws_lock);
+    hipError_t e = hipSuccess;
+    if (!g_rws.done) e = hipEventCreateWithFlags(&g_rws.done, hipEventDisableTiming);
+    if (e == hipSuccess && bytesA + bytesB > g_rws.cap) {
+        e = hipEventSynchronize(g_rws.done);
+        if (e == hipSuccess && g_rws.p) e = hipFree(g_rws.p);
+        g_rws.p = nullptr;
+        g_rws.cap = 0;
+        if (e == hipSuccess) e = hipMalloc(&g_rws.p, bytesA + bytesB);
+        if (e == hipSuccess) g_rws.cap = bytesA + bytesB;
     }
-    int rc;
-    switch (ta * 2 + tb) {
-    case 0: rc = launch_dgemm_kt<MAJ_MN, MAJ_K>(P, S2, st); break;
-    case 1: rc = launch_dgemm_kt<MAJ_MN, MAJ_MN>(P, S2, st); break;
-    case 2: rc = launch_dgemm_kt<MAJ_K, MAJ_K>(P, S2, st); break;
-    default: rc = launch_dgemm_kt<MAJ_K, MAJ_MN>(P, S2, st); break;
-    }
-    if (ws) {
-        hipError_t e = hipEventRecord(g_rws.done, st);
+    if (e == hipSuccess) e = hipStreamWaitEvent(st, g_rws.done, 0);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         pthread_mutex_unlock(&g_rws_lock);
-        if (!rc && e != hipSuccess) rc = fail("ragged dgemm event", e);
+        return fail("dgemm workspace", e);
     }
+    double *wa = (double *)g_rws.p, *wb = (double *)((char *)g_rws.p + bytesA);
+    if (!okA) {
+        launch_repack((const double *)S.A, S.lda, wa, lda2, ra, ca, st);
+        S2.A = wa;
+        S2.lda = lda2;
+    }
+    if (!okB) {
+        launch_repack((const double *)S.B, S.ldb, wb, ldb2, rb, cb, st);
+        S2.B = wb;
+        S2.ldb = ldb2;
+    }
+    int rc = bxh_gemm_tile(BLASX_D, &P, &S2, st);
+    e = hipEventRecord(g_rws.done, st);
+    pthread_mutex_unlock(&g_rws_lock);
+    if (!rc && e != hipSuccess) rc = fail("dgemm workspace event", e);
     return rc ? rc : 1;
-}
-
-template <int MAJA, int MAJB>
-int launch_sgemm_dma(const bxh_problem_t &P, const bxh_seg_t &S, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_sgemm_dma<MAJA, MAJB>), dim3(P.tiles_m * P.tiles_n), dim3(NT), 0, st, P,
-                       S);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : fail("sgemm dma launch", e);
-}
-
-template <typename E> int dispatch_real(int opa, int opb, const bxh_problem_t &P, const bxh_seg_t &S,
-                                        hipStream_t st)
-{
-    const int ta = opa != 0, tb = opb != 0;
-    if constexpr (sizeof(E) == 4) {
-        if (P.m % dmas::BM == 0 && P.n % dmas::BM == 0 && S.k >= dmas::BK &&
-            S.k % dmas::BK == 0 && aligned16(S.A, S.lda, 4) && aligned16(S.B, S.ldb, 4)) {
-            switch (ta * 2 + tb) {
-            case 0: return launch_sgemm_dma<MAJ_MN, MAJ_K>(P, S, st);
-            case 1: return launch_sgemm_dma<MAJ_MN, MAJ_MN>(P, S, st);
-            case 2: return launch_sgemm_dma<MAJ_K, MAJ_K>(P, S, st);
-            default: return launch_sgemm_dma<MAJ_K, MAJ_MN>(P, S, st);
-            }
-        }
-    }
-    if constexpr (sizeof(E) == 8) {
-        if (dgemm_dma_ok(P, S)) {
-            switch (ta * 2 + tb) {
-            case 0: return launch_dgemm_dma<MAJ_MN, MAJ_K>(P, S, st);
-            case 1: return launch_dgemm_dma<MAJ_MN, MAJ_MN>(P, S, st);
-            case 2: return launch_dgemm_dma<MAJ_K, MAJ_K>(P, S, st);
-            default: return launch_dgemm_dma<MAJ_K, MAJ_MN>(P, S, st);
-            }
-        }
-        const int r = dgemm_ragged(ta, tb, P, S, st);
-        if (r != 0) return r < 0 ? r : 0;
-    }
-    switch (ta * 2 + tb) {
-    case 0: return launch_plain<E, MAJ_MN, MAJ_K, false, false>(P, S, st);
-    case 1: return launch_plain<E, MAJ_MN, MAJ_MN, false, false>(P, S, st);
-    case 2: return launch_plain<E, MAJ_K, MAJ_K, false, false>(P, S, st);
-    default: return launch_plain<E, MAJ_K, MAJ_MN, false, false>(P, S, st);
-    }
-}
-
-template <int MAJA, int MAJB, bool CJA, bool CJB>
-int launch_zgemm_dma(const bxh_problem_t &P, const bxh_seg_t &S, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_zgemm_dma<MAJA, MAJB, CJA, CJB>), dim3(P.tiles_m * P.tiles_n), dim3(NT),
-                       0, st, P, S);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : fail("zgemm dma launch", e);
-}
-
-int dispatch_cplx(int opa, int opb, const bxh_problem_t &P, const bxh_seg_t &S, hipStream_t st)
-{
-    // the DMA-staged kernel: no edge tiles, 16-byte aligned operands
-    if (P.m % dmaz::BM == 0 && P.n % dmaz::BN == 0 && S.k >= dmaz::BK && S.k % dmaz::BK == 0 &&
-        aligned16(S.A, S.lda, 16) && aligned16(S.B, S.ldb, 16)) {
-        switch (opa * 3 + opb) {
-        case 0: return launch_zgemm_dma<MAJ_MN, MAJ_K, false, false>(P, S, st);
-        case 1: return launch_zgemm_dma<MAJ_MN, MAJ_MN, false, false>(P, S, st);
-        case 2: return launch_zgemm_dma<MAJ_MN, MAJ_MN, false, true>(P, S, st);
-        case 3: return launch_zgemm_dma<MAJ_K, MAJ_K, false, false>(P, S, st);
-        case 4: return launch_zgemm_dma<MAJ_K, MAJ_MN, false, false>(P, S, st);
-        case 5: return launch_zgemm_dma<MAJ_K, MAJ_MN, false, true>(P, S, st);
-        case 6: return launch_zgemm_dma<MAJ_K, MAJ_K, true, false>(P, S, st);
-        case 7: return launch_zgemm_dma<MAJ_K, MAJ_MN, true, false>(P, S, st);
-        default: return launch_zgemm_dma<MAJ_K, MAJ_MN, true, true>(P, S, st);
-        }
-    }
-    switch (opa * 3 + opb) {
-    case 0: return launch_plain<cplx, MAJ_MN, MAJ_K, false, false>(P, S, st);
-    case 1: return launch_plain<cplx, MAJ_MN, MAJ_MN, false, false>(P, S, st);
-    case 2: return launch_plain<cplx, MAJ_MN, MAJ_MN, false, true>(P, S, st);
-    case 3: return launch_plain<cplx, MAJ_K, MAJ_K, false, false>(P, S, st);
-    case 4: return launch_plain<cplx, MAJ_K, MAJ_MN, false, false>(P, S, st);
-    case 5: return launch_plain<cplx, MAJ_K, MAJ_MN, false, true>(P, S, st);
-    case 6: return launch_plain<cplx, MAJ_K, MAJ_K, true, false>(P, S, st);
-    case 7: return launch_plain<cplx, MAJ_K, MAJ_MN, true, false>(P, S, st);
-    default: return launch_plain<cplx, MAJ_K, MAJ_MN, true, true>(P, S, st);
-    }
 }
 
 } // namespace
@@ -1979,7 +1666,7 @@ int bxh_gemm(int dtype, int opa, int opb, int m, int n, int k, const double *alp
     P.tri = 0;
     P.tri_off = 0;
     P.shape = BXH_SHAPE_128x128;
-    P.pad0 = 0;
+    P.form = 0; /* set per operand alignment (bxh_gemm_tile) */
     bxh_seg_t S;
     S.A = A;
     S.B = B;
@@ -1987,12 +1674,13 @@ int bxh_gemm(int dtype, int opa, int opb, int m, int n, int k, const double *alp
     S.ldb = ldb;
     S.k = k;
     hipStream_t st = (hipStream_t)stream;
-    switch (dtype) {
-    case BLASX_D: return dispatch_real<double>(opa, opb, P, S, st);
-    case BLASX_S: return dispatch_real<float>(opa, opb, P, S, st);
-    case BLASX_Z: return dispatch_cplx(opa, opb, P, S, st);
-    default: return BLASX_EINVAL;
+    if (dtype != BLASX_S && dtype != BLASX_D && dtype != BLASX_Z) return BLASX_EINVAL;
+    if (dtype == BLASX_D) {
+        const int r = dgemm_repacked(opa != 0, opb != 0, P, S, st);
+        if (r) return r < 0 ? r : 0;
     }
+    const int rc = bxh_gemm_tile(dtype, &P, &S, st);
+    return rc ? fail("gemm launch", hipErrorLaunchFailure) : 0;
 }
 
 int bxh_gemm_grouped(int dtype, const bxh_problem_t *probs_dev, int nprob,

@@ -45,10 +45,15 @@ typedef struct bxh_problem {
     int32_t tri, tri_off;
     /* block tile shape (real types): 0 = 128 x 128, 1 = 128 x 64, 2 = 64 x 64
      * (BXH_SHAPE_*); complex problems use 0 (128 x 64 complex) */
-    int32_t shape, pad0;
+    int32_t shape;
+    int32_t form; /* how the operands are moved (BXH_FORM_*) */
     double alpha_re, alpha_im;
     double beta_re, beta_im;
 } bxh_problem_t;
+
+#define BXH_FORM_DMA 0     /* 16-byte aligned operands: global memory to LDS */
+#define BXH_FORM_REG 1     /* through registers, at element alignment */
+#define BXH_FORM_ELEMENT 2 /* element by element, any operands */
 
 #define BX_TRI_LOWER 1
 #define BX_TRI_UPPER 2
@@ -110,6 +115,11 @@ int bxh_graph_destroy(void *exec);
 int bxh_gemm(int dtype, int opa, int opb, int m, int n, int k, const double *alpha,
              const void *A, int64_t lda, const void *B, int64_t ldb, const double *beta,
              void *C, int64_t ldc, void *stream);
+/* one problem on the block tile shape and operand movement that run it
+ * fastest (hip/gemm_tiles.hip) */
+int bxh_tile_form(int dtype, int opa, int opb, int m, int n, const void *A, int64_t lda,
+                  const void *B, int64_t ldb);
+int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *stream);
 /* grouped launch over a device-resident problem and segment table; all
  * problems share dtype.  grid = 0 picks one block per tile. */
 int bxh_gemm_grouped(int dtype, const bxh_problem_t *probs_dev, int nprob,
