@@ -14,6 +14,7 @@
 #include <string.h>
 
 #include "internal.h"
+#include "tilecost.h"
 
 static int op_of(int dt, int t)
 {
@@ -42,20 +43,95 @@ static int desc_runs(const blasx_gemm_desc_t *x, int dtype)
     return x->K != 0 && !az;
 }
 
+/* exchange two table entries (each problem has one segment) */
+static void swap_entries(bxh_problem_t *probs, bxh_seg_t *segs, int i, int j)
+{
+    const bxh_problem_t p = probs[i];
+    const bxh_seg_t s = segs[i];
+    probs[i] = probs[j];
+    segs[i] = segs[j];
+    probs[j] = p;
+    segs[j] = s;
+}
+
+/* restore the heap (least K at the root) of n entries below entry r */
+static void sift(bxh_problem_t *probs, bxh_seg_t *segs, int r, int n)
+{
+    for (int c; (c = 2 * r + 1) < n; r = c) {
+        if (c + 1 < n && segs[c + 1].k < segs[c].k) ++c;
+        if (segs[r].k <= segs[c].k) return;
+        swap_entries(probs, segs, r, c);
+    }
+}
+
+/* Longest tiles first, so that the short ones fill the last wave: descending
+ * K, by heap sort (in place: this path may not allocate).  Equal problems,
+ * the usual launch, are left as they are. */
+static void sort_by_k(bxh_problem_t *probs, bxh_seg_t *segs, int n)
+{
+    int sorted = 1;
+    for (int i = 1; i < n && sorted; ++i) sorted = segs[i - 1].k >= segs[i].k;
+    if (sorted) return;
+    for (int r = n / 2 - 1; r >= 0; --r) sift(probs, segs, r, n);
+    for (int end = n - 1; end > 0; --end) {
+        swap_entries(probs, segs, 0, end);
+        sift(probs, segs, 0, end);
+    }
+}
+
+/* 64x64 tiles or 32x32 ones for the n problems of one launch: whichever
+ * spreads over the CUs in less time, the tiles' total over 256 CUs plus half
+ * the longest (what longest-first order leaves uneven), tilecost.h */
+static int small_shape(int dtype, const bxh_problem_t *probs, const bxh_seg_t *segs, int n)
+{
+    double t[2];
+    const int s[2] = {BXC_64x64, BXC_32x32};
+    for (int j = 0; j < 2; ++j) {
+        double sum = 0, most = 0;
+        for (int i = 0; i < n; ++i) {
+            const bx_cost_t *c = probs[i].form == BXH_FORM_DMA ? &BX_COST_DMA[dtype][s[j]]
+                                                               : &BX_COST_REG[dtype][s[j]];
+            const double one = bx_cost_tile(c, segs[i].k);
+            sum += one * (double)bx_cost_tiles(s[j], probs[i].m, probs[i].n);
+            if (one > most) most = one;
+        }
+        t[j] = sum / 256 + 0.5 * most;
+    }
+    return t[1] < t[0] ? BXH_SHAPE_32x32 : BXH_SHAPE_64x64;
+}
+
+/* tile counts and starts of problems [first, first + n), from 0 */
+static int place_tiles(int dtype, bxh_problem_t *probs, int n)
+{
+    int total = 0;
+    for (int i = 0; i < n; ++i) {
+        int bm, bn;
+        bxh_tile_dims(dtype, probs[i].shape, &bm, &bn);
+        probs[i].tiles_m = (probs[i].m + bm - 1) / bm;
+        probs[i].tiles_n = (probs[i].n + bn - 1) / bn;
+        probs[i].tile_start = total;
+        total += probs[i].tiles_m * probs[i].tiles_n;
+    }
+    return total;
+}
+
 /* Fill problem/segment tables for the descriptors of one dtype (device
  * pointers in the descriptors).  Descriptors with alpha == 0 or K == 0 are
- * skipped (the caller scales C separately).  Each problem's block tile
- * shape comes from bx_grouped_shape, given the launch's load: its tile
- * count at the large tile.  Returns the tile total. */
-int bx_grouped_fill(const blasx_gemm_desc_t *d, int n, int dtype, bxh_problem_t *probs,
-                    bxh_seg_t *segs, int *nprob)
+ * skipped (the caller scales C separately).  Each real problem's shape comes
+ * from bx_grouped_shape, given the launch's load: its tile count at the large
+ * tile; problems on 64x64 tiles, complex ones and those whose operands do
+ * not take the DMA share one choice of 64x64 or 32x32.  The first nprob[0]
+ * problems (total[0] tiles) are those, the next nprob[1] (total[1] tiles, a
+ * launch of their own) the 128-row shapes; big = 0 puts all in the first. */
+void bx_grouped_fill(const blasx_gemm_desc_t *d, int n, int dtype, bxh_problem_t *probs,
+                     bxh_seg_t *segs, int big, int nprob[2], int total[2])
 {
     const int bm0 = bxh_tile_m(dtype), bn0 = bxh_tile_n(dtype);
     int64_t load = 0;
     for (int i = 0; i < n; ++i)
         if (desc_runs(&d[i], dtype))
             load += (int64_t)((d[i].M + bm0 - 1) / bm0) * ((d[i].N + bn0 - 1) / bn0);
-    int np = 0, total = 0;
+    int np = 0, nbig = 0;
     /* the previous problem's choice, reused while M, N and K repeat: the
      * table lookup takes a lock and interpolates, which on launches of many
      * small equal problems cost more host time than the kernel took */
@@ -64,28 +140,20 @@ int bx_grouped_fill(const blasx_gemm_desc_t *d, int n, int dtype, bxh_problem_t 
         const blasx_gemm_desc_t *x = &d[i];
         if (!desc_runs(x, dtype)) continue;
         bxh_problem_t *P = &probs[np];
-        int bm, bn;
         if (x->M != lm || x->N != ln || x->K != lk) {
             shape = bx_grouped_shape(dtype, x->M, x->N, x->K, load);
             lm = x->M;
             ln = x->N;
             lk = x->K;
         }
-        bxh_tile_dims(dtype, shape, &bm, &bn);
         memset(P, 0, sizeof *P);
         P->C = x->C;
         P->ldc = x->ldc;
         P->m = x->M;
         P->n = x->N;
         P->nseg = 1;
-        P->seg_off = np;
         P->opa = op_of(dtype, x->transa);
         P->opb = op_of(dtype, x->transb);
-        P->shape = shape;
-        P->tiles_m = (x->M + bm - 1) / bm;
-        P->tiles_n = (x->N + bn - 1) / bn;
-        P->tile_start = total;
-        total += P->tiles_m * P->tiles_n;
         P->alpha_re = x->alpha[0];
         P->alpha_im = dtype == BLASX_Z ? x->alpha[1] : 0.0;
         P->beta_re = x->beta[0];
@@ -96,18 +164,63 @@ int bx_grouped_fill(const blasx_gemm_desc_t *d, int n, int dtype, bxh_problem_t 
         segs[np].lda = x->lda;
         segs[np].ldb = x->ldb;
         segs[np].k = x->K;
+        P->form = bxh_tile_form(dtype, P->opa, P->opb, P->m, P->n, &segs[np]);
+        P->shape = big && dtype != BLASX_Z && P->form == BXH_FORM_DMA ? shape : BXH_SHAPE_64x64;
+        /* small problems stay in front of the big ones */
+        if (P->shape != BXH_SHAPE_64x64)
+            ++nbig;
+        else if (nbig)
+            swap_entries(probs, segs, np, np - nbig);
         ++np;
     }
-    *nprob = np;
-    return total;
+    const int ns = np - nbig;
+    if (ns) {
+        const int s = small_shape(dtype, probs, segs, ns);
+        for (int i = 0; i < ns; ++i) probs[i].shape = s;
+    }
+    sort_by_k(probs, segs, ns);
+    sort_by_k(probs + ns, segs + ns, nbig);
+    for (int i = 0; i < np; ++i) probs[i].seg_off = i;
+    nprob[0] = ns;
+    nprob[1] = nbig;
+    total[0] = place_tiles(dtype, probs, ns);
+    total[1] = place_tiles(dtype, probs + ns, nbig);
+}
+
+/* the launches of one dtype's tables */
+static int launch_tables(int dtype, const bxh_problem_t *probs, const bxh_seg_t *segs,
+                         const int nprob[2], const int total[2], void *st, int *launches)
+{
+    int rc = 0;
+    if (nprob[0]) {
+        rc = bxh_gemm_grouped(dtype, probs, nprob[0], segs, total[0], 0, st);
+        ++*launches;
+    }
+    if (!rc && nprob[1]) {
+        rc = bxh_gemm_grouped(dtype, probs + nprob[0], nprob[1], segs, total[1], BXH_GROUP_BIG, st);
+        ++*launches;
+    }
+    return rc;
+}
+
+static double desc_flops(const blasx_gemm_desc_t *d, int n, int dtype)
+{
+    double f = 0;
+    for (int i = 0; i < n; ++i)
+        if (d[i].dtype == dtype)
+            f += (dtype == BLASX_Z ? 8.0 : 2.0) * d[i].M * (double)d[i].N * d[i].K;
+    return f;
 }
 
 /* ---- blasx_gemm_grouped_device ---- */
+/* table staging: the host runs up to GRING calls ahead of the GPU */
+enum { GRING = 4 };
 static pthread_mutex_t g_glock = PTHREAD_MUTEX_INITIALIZER;
 static struct {
     void *host, *dev, *done;
     size_t cap;
-} g_gbuf;
+} g_gring[GRING];
+static unsigned g_gnext;
 
 BX_EXPORT int blasx_gemm_grouped_device(const blasx_gemm_desc_t *d, int n, void *stream)
 {
@@ -125,42 +238,44 @@ BX_EXPORT int blasx_gemm_grouped_device(const blasx_gemm_desc_t *d, int n, void 
     }
     if (rc || n == 0) return rc;
 
-    const size_t per = (size_t)n * (sizeof(bxh_problem_t) + sizeof(bxh_seg_t));
-    const size_t need = 3 * ((per + 255) & ~(size_t)255);
+    /* one table entry per descriptor, whatever its type: problems, then segments */
+    const size_t seg_at = (size_t)n * sizeof(bxh_problem_t);
+    const size_t need = seg_at + (size_t)n * sizeof(bxh_seg_t);
     pthread_mutex_lock(&g_glock);
-    if (!g_gbuf.done) rc = bxh_event_create(&g_gbuf.done, 0);
-    if (!rc) rc = bxh_event_sync(g_gbuf.done); /* the staging buffers are free again */
-    if (!rc && need > g_gbuf.cap) {
-        bxh_host_free(g_gbuf.host);
-        bxh_free(g_gbuf.dev);
-        g_gbuf.host = g_gbuf.dev = NULL;
-        g_gbuf.cap = 0;
-        rc = bxh_host_malloc(&g_gbuf.host, need);
-        if (!rc) rc = bxh_malloc(&g_gbuf.dev, need);
-        if (!rc) g_gbuf.cap = need;
+    const unsigned slot = g_gnext++ % GRING;
+    if (!g_gring[slot].done) rc = bxh_event_create(&g_gring[slot].done, 0);
+    if (!rc) rc = bxh_event_sync(g_gring[slot].done); /* this slot's tables are consumed */
+    if (!rc && need > g_gring[slot].cap) {
+        bxh_host_free(g_gring[slot].host);
+        bxh_free(g_gring[slot].dev);
+        g_gring[slot].host = g_gring[slot].dev = NULL;
+        g_gring[slot].cap = 0;
+        rc = bxh_host_malloc(&g_gring[slot].host, need);
+        if (!rc) rc = bxh_malloc(&g_gring[slot].dev, need);
+        if (!rc) g_gring[slot].cap = need;
     }
     const int dts[3] = {BLASX_S, BLASX_D, BLASX_Z};
-    const size_t slot = (per + 255) & ~(size_t)255;
-    int launches = 0;
+    int np[3][2] = {{0}}, total[3][2] = {{0}}, first[3], used = 0, launches = 0;
     double flops = 0;
-    for (int k = 0; k < 3 && !rc; ++k) {
-        char *h = (char *)g_gbuf.host + k * slot, *dv = (char *)g_gbuf.dev + k * slot;
-        bxh_problem_t *probs = (bxh_problem_t *)h;
-        bxh_seg_t *segs = (bxh_seg_t *)(h + (size_t)n * sizeof(bxh_problem_t));
-        int np = 0;
-        const int total = bx_grouped_fill(d, n, dts[k], probs, segs, &np);
-        if (np == 0) continue;
-        rc = bxh_memcpy_h2d_async(dv, h, per, st);
-        if (!rc)
-            rc = bxh_gemm_grouped(dts[k], (const bxh_problem_t *)dv, np,
-                                  (const bxh_seg_t *)(dv + (size_t)n * sizeof(bxh_problem_t)),
-                                  total, 0, st);
-        ++launches;
-        for (int i = 0; i < n; ++i)
-            if (d[i].dtype == dts[k])
-                flops += (dts[k] == BLASX_Z ? 8.0 : 2.0) * d[i].M * (double)d[i].N * d[i].K;
+    if (!rc) {
+        bxh_problem_t *probs = (bxh_problem_t *)g_gring[slot].host;
+        bxh_seg_t *segs = (bxh_seg_t *)((char *)g_gring[slot].host + seg_at);
+        for (int k = 0; k < 3; ++k) {
+            first[k] = used;
+            bx_grouped_fill(d, n, dts[k], probs + used, segs + used, 1, np[k], total[k]);
+            used += np[k][0] + np[k][1];
+            flops += desc_flops(d, n, dts[k]);
+        }
+        if (used) rc = bxh_memcpy_h2d_async(g_gring[slot].dev, g_gring[slot].host, need, st);
     }
-    if (!rc) rc = bxh_event_record(g_gbuf.done, st);
+    for (int k = 0; k < 3 && !rc; ++k)
+        rc = launch_tables(dts[k], (const bxh_problem_t *)g_gring[slot].dev + first[k],
+                           (const bxh_seg_t *)((char *)g_gring[slot].dev + seg_at) + first[k], np[k],
+                           total[k], st, &launches);
+    if (g_gring[slot].done) {
+        const int re = bxh_event_record(g_gring[slot].done, st);
+        if (!rc) rc = re;
+    }
     pthread_mutex_unlock(&g_glock);
     if (!rc) {
         BX_STAT_ADD(kernel_launches, launches);
@@ -218,20 +333,19 @@ BX_EXPORT int blasx_gemm_grouped_device_noalloc(const blasx_gemm_desc_t *d, int 
         char *dv = (char *)store + (size_t)k * BXH_NOALLOC_SLOT_BYTES;
         bxh_problem_t *probs = (bxh_problem_t *)h;
         bxh_seg_t *segs = (bxh_seg_t *)(h + BXH_NOALLOC_SEG_OFFSET);
-        int np = 0;
-        const int total = bx_grouped_fill(d, n, dts[k], probs, segs, &np);
+        int nprob[2], total[2];
+        bx_grouped_fill(d, n, dts[k], probs, segs, 1, nprob, total);
+        const size_t np = (size_t)(nprob[0] + nprob[1]);
         if (np == 0) continue;
-        rc = bxh_memcpy_h2d_async(dv, h, (size_t)np * sizeof(bxh_problem_t), st);
+        rc = bxh_memcpy_h2d_async(dv, h, np * sizeof(bxh_problem_t), st);
         if (!rc)
             rc = bxh_memcpy_h2d_async(dv + BXH_NOALLOC_SEG_OFFSET, h + BXH_NOALLOC_SEG_OFFSET,
-                                      (size_t)np * sizeof(bxh_seg_t), st);
+                                      np * sizeof(bxh_seg_t), st);
         if (!rc)
-            rc = bxh_gemm_grouped(dts[k], (const bxh_problem_t *)dv, np,
-                                  (const bxh_seg_t *)(dv + BXH_NOALLOC_SEG_OFFSET), total, 0, st);
-        ++launches;
-        for (int i = 0; i < n; ++i)
-            if (d[i].dtype == dts[k])
-                flops += (dts[k] == BLASX_Z ? 8.0 : 2.0) * d[i].M * (double)d[i].N * d[i].K;
+            rc = launch_tables(dts[k], (const bxh_problem_t *)dv,
+                               (const bxh_seg_t *)(dv + BXH_NOALLOC_SEG_OFFSET), nprob, total, st,
+                               &launches);
+        flops += desc_flops(d, n, dts[k]);
     }
     if (!rc) rc = bxh_event_record(g_na_copied, st);
     if (!rc) rc = bxh_event_record(done, st);

@@ -82,6 +82,78 @@ __host__ __device__ __forceinline__ bool aligned16(const void *p, int64_t ld, in
     return ((reinterpret_cast<uintptr_t>(p) & 15) == 0) && (((ld * esize) & 15) == 0);
 }
 
+// Tile loc of a group of `rows` tile rows and `cols` tile columns, walked so
+// that all XCDs (block b runs on XCD b % 8) are on the same rows, each on
+// columns of its own: the rows' operand panels come from the Infinity Cache
+// whatever K each block has reached, and a column's panel is read by the
+// `rows` blocks that one XCD runs one after the other.
+__host__ __device__ __forceinline__ void striped(int64_t loc, int rows, int cols, int &r, int &c)
+{
+    const int full = cols & ~7;
+    const int64_t nf = (int64_t)rows * full;
+    if (loc < nf) {
+        const int64_t q = loc >> 3;
+        r = (int)(q % rows);
+        c = (int)(q / rows) * 8 + (int)(loc & 7);
+    } else {
+        const int w = cols - full;
+        r = (int)((loc - nf) / w);
+        c = full + (int)((loc - nf) % w);
+    }
+}
+template <int G>
+__device__ __forceinline__ void tile_coords_striped(int t, int tiles_m, int tiles_n, int &tm, int &tn)
+{
+    const int64_t per = (int64_t)G * tiles_n;
+    const int g = (int)(t / per), rows = min(tiles_m - g * G, G);
+    int r;
+    striped(t - g * per, rows, tiles_n, r, tn);
+    tm = g * G + r;
+}
+
+// The tiles of a rank-k update's stored triangle, G tile rows at a time, each
+// group striped over the XCDs: group g has its first tri_cols(g) tile columns
+// (for an upper triangle, both counted from the last).  The few tiles of a
+// group beyond the diagonal are skipped by the kernel.
+template <int G, int BM, int BN> __host__ __device__ __forceinline__ int64_t tri_cols(int64_t g, int tiles_n)
+{
+    static_assert(BM % BN == 0, "whole columns per row");
+    const int64_t c = (BM / BN) * G * (g + 1) + 1;
+    return c < tiles_n ? c : tiles_n;
+}
+// tiles before group g (only the last group's columns can be clipped: a group
+// before it ends at least one column short of the last)
+template <int G, int BM, int BN> __host__ __device__ __forceinline__ int64_t tri_before(int64_t g)
+{
+    return G * ((BM / BN) * G * (g * (g + 1) / 2) + g);
+}
+template <int G, int BM, int BN>
+__host__ __device__ __forceinline__ int64_t tri_tiles(int tiles_m, int tiles_n)
+{
+    const int64_t last = (tiles_m - 1) / G;
+    return tri_before<G, BM, BN>(last) + (tiles_m - last * G) * tri_cols<G, BM, BN>(last, tiles_n);
+}
+template <int G, int BM, int BN>
+__host__ __device__ __forceinline__ void tri_coords(int64_t t, int upper, int tiles_m, int tiles_n,
+                                                    int &tm, int &tn)
+{
+    // g: the last group that starts at or before t
+    const double r = (BM / BN) * (double)G * G, h = r / 2 + G;
+    int64_t g = (int64_t)((sqrt(h * h + 2 * r * (double)t) - h) / r);
+    while (g > 0 && tri_before<G, BM, BN>(g) > t) --g;
+    while (tri_before<G, BM, BN>(g + 1) <= t) ++g;
+    const int64_t last = (tiles_m - 1) / G;
+    if (g > last) g = last;
+    const int rows = (int)(tiles_m - g * G < G ? tiles_m - g * G : G);
+    int row;
+    striped(t - tri_before<G, BM, BN>(g), rows, (int)tri_cols<G, BM, BN>(g, tiles_n), row, tn);
+    tm = (int)g * G + row;
+    if (upper) {
+        tm = tiles_m - 1 - tm;
+        tn = tiles_n - 1 - tn;
+    }
+}
+
 // block tile index -> (tm, tn), walking groups of 8 tile rows so that the
 // blocks resident at one time share A row panels and B column panels
 template <int G = 8>
@@ -96,15 +168,23 @@ __device__ __forceinline__ void tile_coords(int t, int tiles_m, int tiles_n, int
     tn = r / gsz;
 }
 
-// segment i of the table, or the by-value segment when there is no table;
+// segment i of the table, or of the by-value pair when there is no table;
 // fields are read through the global address space one by one (selecting
 // between a table pointer and a local would make every access FLAT)
-__device__ __forceinline__ bxh_seg_t seg_at(const bxh_seg_t *segs, const bxh_seg_t &seg0, int i)
+__device__ __forceinline__ bxh_seg_t seg_at(const bxh_seg_t *segs, const bxh_seg_t &seg0,
+                                            const bxh_seg_t &seg1, int i)
 {
-    if (!segs) return seg0;
+    bxh_seg_t s;
+    if (!segs) {
+        s.A = i ? seg1.A : seg0.A;
+        s.B = i ? seg1.B : seg0.B;
+        s.lda = i ? seg1.lda : seg0.lda;
+        s.ldb = i ? seg1.ldb : seg0.ldb;
+        s.k = i ? seg1.k : seg0.k;
+        return s;
+    }
     const __attribute__((address_space(1))) bxh_seg_t *g =
         (const __attribute__((address_space(1))) bxh_seg_t *)(segs + i);
-    bxh_seg_t s;
     s.A = g->A;
     s.B = g->B;
     s.lda = g->lda;

@@ -43,8 +43,7 @@ typedef struct bxh_problem {
      * row + tri_off <= col (row, col relative to C); BX_TRI_HERM also zeroes
      * the imaginary part where row + tri_off == col.  0: every element. */
     int32_t tri, tri_off;
-    /* block tile shape (real types): 0 = 128 x 128, 1 = 128 x 64, 2 = 64 x 64
-     * (BXH_SHAPE_*); complex problems use 0 (128 x 64 complex) */
+    /* block tile shape (BXH_SHAPE_*) */
     int32_t shape;
     int32_t form; /* how the operands are moved (BXH_FORM_*) */
     double alpha_re, alpha_im;
@@ -65,7 +64,8 @@ int bxh_tile_n(int dtype);
 #define BXH_SHAPE_128x128 0
 #define BXH_SHAPE_128x64 1
 #define BXH_SHAPE_64x64 2
-#define BXH_NSHAPES 3
+#define BXH_NSHAPES 3 /* shapes a caller can ask for; below: finer cuts of 64 x 64 */
+#define BXH_SHAPE_32x32 3
 /* block-tile edges of a grouped problem of this element type and shape */
 void bxh_tile_dims(int dtype, int shape, int *bm, int *bn);
 
@@ -115,17 +115,34 @@ int bxh_graph_destroy(void *exec);
 int bxh_gemm(int dtype, int opa, int opb, int m, int n, int k, const double *alpha,
              const void *A, int64_t lda, const void *B, int64_t ldb, const double *beta,
              void *C, int64_t ldc, void *stream);
-/* one problem on the block tile shape and operand movement that run it
- * fastest (hip/gemm_tiles.hip) */
-int bxh_tile_form(int dtype, int opa, int opb, int m, int n, const void *A, int64_t lda,
-                  const void *B, int64_t ldb);
+/* How a problem's operands are moved (one segment of it): by DMA when both
+ * are 16-byte aligned, else through registers at element alignment; element
+ * by element where not even one 16-byte load fits a row-contiguous operand's
+ * column, or a leading dimension is beyond the movers' 32-bit offsets. */
+static inline int bxh_tile_form(int dtype, int opa, int opb, int m, int n, const bxh_seg_t *s)
+{
+    const int es = dtype == 0 ? 4 : dtype == 1 ? 8 : 16;
+    const int64_t most = ((int64_t)1 << 32) / (8 * es) - 1024;
+    if (s->lda >= most || s->ldb >= most) return BXH_FORM_ELEMENT;
+    if (((uintptr_t)s->A & 15) == 0 && ((uintptr_t)s->B & 15) == 0 && (s->lda * es & 15) == 0 &&
+        (s->ldb * es & 15) == 0)
+        return BXH_FORM_DMA;
+    if ((opa == 0 && m < 16 / es) || (opb != 0 && n < 16 / es)) return BXH_FORM_ELEMENT;
+    return BXH_FORM_REG;
+}
+/* one problem of one or two K segments (S[0 .. nseg)), or a rank-k update's
+ * stored triangle (tri, m == n), on the block tile shape that runs it fastest
+ * (hip/gemm_tiles.hip); its form, shape and tile fields are not read */
 int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *stream);
 /* grouped launch over a device-resident problem and segment table; all
- * problems share dtype.  grid = 0 picks one block per tile. */
+ * problems share dtype.  grid = 0: one block per tile, every problem's shape
+ * BXH_SHAPE_64x64 or BXH_SHAPE_32x32; grid = BXH_GROUP_BIG: one block per
+ * tile, every problem real, moved by DMA, of a 128-row shape. */
+#define BXH_GROUP_BIG (-1)
 int bxh_gemm_grouped(int dtype, const bxh_problem_t *probs_dev, int nprob,
                      const bxh_seg_t *segs_dev, int total_tiles, int grid, void *stream);
-/* persistent grouped launch for graph replay: counts_dev[0] = nprob,
- * counts_dev[1] = total tiles, both read by the kernel */
+/* persistent grouped launch for graph replay (64x64 and 32x32 tiles):
+ * counts_dev[0] = nprob, counts_dev[1] = total tiles, both read by the kernel */
 int bxh_gemm_grouped_dyn(int dtype, const bxh_problem_t *probs_dev, const bxh_seg_t *segs_dev,
                          const int *counts_dev, int grid, void *stream);
 /* C = beta * C (beta == 0 writes zeros without reading C) */

@@ -154,8 +154,8 @@ int bx_autotune_tile(int dt, int M, int N, int K);
 
 /* grouped GEMM tables (grouped.c) */
 int bx_desc_check(const blasx_gemm_desc_t *d);
-int bx_grouped_fill(const blasx_gemm_desc_t *d, int n, int dtype, bxh_problem_t *probs,
-                    bxh_seg_t *segs, int *nprob);
+void bx_grouped_fill(const blasx_gemm_desc_t *d, int n, int dtype, bxh_problem_t *probs,
+                     bxh_seg_t *segs, int big, int nprob[2], int total[2]);
 /* block tile shape (BXH_SHAPE_*) of a grouped problem in a launch of `load`
  * large tiles of its element type (autotune.c) */
 int bx_grouped_shape(int dt, int M, int N, int K, int64_t load);

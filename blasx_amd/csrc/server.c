@@ -255,10 +255,10 @@ static int launch_batch(blasx_server_t *s, batch_t *b)
         char *p = slot_part(s, (char *)b->desc_host, k);
         bxh_problem_t *probs = (bxh_problem_t *)(p + 256);
         bxh_seg_t *segs = (bxh_seg_t *)(p + 256 + (size_t)s->max_batch * sizeof(bxh_problem_t));
-        int np = 0;
-        const int total = bx_grouped_fill(dev, b->n, dts[k], probs, segs, &np);
-        ((int *)p)[0] = np;
-        ((int *)p)[1] = total;
+        int np[2], total[2];
+        bx_grouped_fill(dev, b->n, dts[k], probs, segs, 0, np, total);
+        ((int *)p)[0] = np[0];
+        ((int *)p)[1] = total[0];
     }
     if (!rc) rc = bxh_memcpy_h2d_async(b->desc_dev, b->desc_host, 3 * s->slot_bytes, s->s_comp);
     for (int i = 0; i < b->n && !rc; ++i) {
@@ -431,7 +431,7 @@ BX_EXPORT blasx_server_t *blasx_server_create(size_t hbm_bytes, int max_batch)
     pthread_cond_init(&s->cv_work, NULL);
     pthread_cond_init(&s->cv_done, NULL);
     s->max_batch = max_batch;
-    s->grid = 2 * (g_bx.cus > 0 ? g_bx.cus : 256);
+    s->grid = 3 * (g_bx.cus > 0 ? g_bx.cus : 256);
     s->slot_bytes = (256 + (size_t)max_batch * (sizeof(bxh_problem_t) + sizeof(bxh_seg_t)) + 255) &
                     ~(size_t)255;
     int rc = arena_init(&s->arena, hbm_bytes);

@@ -17,15 +17,13 @@
  * CSYRK and CHERK (complex64) run on the FP32 matrix cores as a full product
  * whose stored triangle is copied back (bx_gpu_crank, level3.c).  For the
  * other types, host operands go through the tile runtime (bx_tile_syrk) and
- * operands in HBM run as one grouped launch here: for each 256-row panel of C, the
- * off-diagonal part is a plain GEMM problem (eligible for the DMA-staged
- * block) and the diagonal 256 x 256 block a masked one.
+ * operands in HBM run as one launch here, over the tiles on the stored
+ * triangle, those on the diagonal masked.
  *
  * Deviations (netlib semantics): RowMajor is computed (the other triangle
  * with the transposition flipped); ZSYRK rejects ConjTrans (info 2), as
  * netlib does; f77 argument errors report the lowest parameter number.
  */
-#include <pthread.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -35,43 +33,6 @@
 #include "internal.h"
 
 /* ---------------------------------------------------------------- device */
-enum { PANEL = 256 };
-
-static pthread_mutex_t g_slock = PTHREAD_MUTEX_INITIALIZER;
-static struct {
-    void *host, *dev, *done;
-    size_t cap;
-} g_sbuf;
-
-/* one problem (C block m x n) with its K segments seg[0..nseg) */
-static void add_problem(bxh_problem_t *P, bxh_seg_t *S, int idx, int nseg, const bxh_seg_t *seg,
-                        int dt, void *C, int64_t ldc, int m, int n, int opa, int opb,
-                        const double *alpha, const double *beta, int tri, int *total)
-{
-    const int bm = bxh_tile_m(dt), bn = bxh_tile_n(dt);
-    memset(P, 0, sizeof *P);
-    P->C = C;
-    P->ldc = ldc;
-    P->m = m;
-    P->n = n;
-    P->nseg = nseg;
-    P->seg_off = idx * nseg;
-    P->opa = opa;
-    P->opb = opb;
-    P->tiles_m = (m + bm - 1) / bm;
-    P->tiles_n = (n + bn - 1) / bn;
-    P->tile_start = *total;
-    *total += P->tiles_m * P->tiles_n;
-    P->alpha_re = alpha[0];
-    P->alpha_im = alpha[1];
-    P->beta_re = beta[0];
-    P->beta_im = beta[1];
-    P->beta_zero = beta[0] == 0.0 && beta[1] == 0.0;
-    P->tri = tri;
-    P->tri_off = 0;
-    for (int i = 0; i < nseg; ++i) S[i] = seg[i];
-}
-
 /* operands, C and the launch on `stream` (NULL: the library's compute
  * stream); asynchronous, like the other device entry points.  With B (SYR2K)
  * C = alpha op(A) op(B)^T + alpha op(B) op(A)^T + beta C on the triangle. */
@@ -95,79 +56,29 @@ int bx_device_syr2k(int dt, int tri, int opa, int N, int K, const double *alpha,
     if (K == 0 || (alpha[0] == 0.0 && alpha[1] == 0.0))
         return bxh_scale_tri(dt, N, N, tri, beta, C, ldc, st);
 
-    const int es = bx_esize(dt);
-    const int opb = opa != BX_OP_N ? BX_OP_N : (tri & BX_TRI_HERM) ? BX_OP_C : BX_OP_T;
-    const int npan = (N + PANEL - 1) / PANEL, maxp = 2 * npan, nseg = B ? 2 : 1;
-    const size_t prob_bytes = ((size_t)maxp * sizeof(bxh_problem_t) + 255) & ~(size_t)255;
-    const size_t need = prob_bytes + (size_t)maxp * nseg * sizeof(bxh_seg_t);
-    int rc = 0;
-    pthread_mutex_lock(&g_slock);
-    if (!g_sbuf.done) rc = bxh_event_create(&g_sbuf.done, 0);
-    if (!rc) rc = bxh_event_sync(g_sbuf.done); /* the previous call's tables are consumed */
-    if (!rc && need > g_sbuf.cap) {
-        bxh_host_free(g_sbuf.host);
-        bxh_free(g_sbuf.dev);
-        g_sbuf.host = g_sbuf.dev = NULL;
-        g_sbuf.cap = 0;
-        rc = bxh_host_malloc(&g_sbuf.host, need);
-        if (!rc) rc = bxh_malloc(&g_sbuf.dev, need);
-        if (!rc) g_sbuf.cap = need;
-    }
+    /* one launch over the tiles on the stored triangle; term 1: op(A) x op(B)^T
+     * (op(A)^T for SYRK), term 2 (SYR2K): op(B2) x op(A)^T */
+    bxh_problem_t P;
+    memset(&P, 0, sizeof P);
+    P.C = C;
+    P.ldc = ldc;
+    P.m = P.n = N;
+    P.nseg = B ? 2 : 1;
+    P.opa = opa;
+    P.opb = opa != BX_OP_N ? BX_OP_N : (tri & BX_TRI_HERM) ? BX_OP_C : BX_OP_T;
+    P.alpha_re = alpha[0];
+    P.alpha_im = alpha[1];
+    P.beta_re = beta[0];
+    P.beta_im = beta[1];
+    P.beta_zero = beta[0] == 0.0 && beta[1] == 0.0;
+    P.tri = tri;
+    const bxh_seg_t S[2] = {{A, B ? B : A, lda, B ? ldb : lda, K},
+                            {B2 ? B2 : B, A, B2 ? ldb2 : ldb, lda, K}};
+    const int rc = bxh_gemm_tile(dt, &P, S, st);
     if (!rc) {
-        bxh_problem_t *probs = (bxh_problem_t *)g_sbuf.host;
-        bxh_seg_t *segs = (bxh_seg_t *)((char *)g_sbuf.host + prob_bytes);
-        const char *a = (const char *)A, *b = B ? (const char *)B : (const char *)A;
-        const char *b2 = B2 ? (const char *)B2 : b;
-        char *c = (char *)C;
-        /* row x of op(A) starts at element x of A (op N) or at column x (T, C) */
-        const int64_t step = (opa == BX_OP_N ? 1 : lda) * es;
-        const int64_t stepb = (opa == BX_OP_N ? 1 : ldb) * es;
-        const int64_t stepb2 = (opa == BX_OP_N ? 1 : ldb2) * es;
-        int np = 0, total = 0;
-        for (int r0 = 0; r0 < N; r0 += PANEL) {
-            const int rows = N - r0 < PANEL ? N - r0 : PANEL;
-            /* rows r0.. of op(C) against columns c0.. (count n) */
-            int c0 = r0, n = rows, with_tri = tri;
-            for (int part = 0; part < 2; ++part) {
-                if (part == 1) {
-                    with_tri = 0;
-                    if (tri & BX_TRI_LOWER)
-                        c0 = 0, n = r0;
-                    else
-                        c0 = r0 + rows, n = N - c0;
-                    if (n <= 0) break;
-                }
-                /* term 1: op(A) rows r0.. x op(B) rows c0..; term 2 (SYR2K): op(B)
-                 * rows r0.. x op(A) rows c0..; SYRK has B = A and one term */
-                bxh_seg_t sg[2];
-                sg[0].A = a + r0 * step;
-                sg[0].lda = lda;
-                sg[0].B = B ? b + c0 * stepb : a + c0 * step;
-                sg[0].ldb = B ? ldb : lda;
-                sg[0].k = K;
-                sg[1].A = b2 + r0 * stepb2;
-                sg[1].lda = B2 ? ldb2 : ldb;
-                sg[1].B = a + c0 * step;
-                sg[1].ldb = lda;
-                sg[1].k = K;
-                add_problem(&probs[np], &segs[np * nseg], np, nseg, sg, dt,
-                            c + (r0 + (int64_t)c0 * ldc) * es, ldc, rows, n, opa, opb, alpha,
-                            beta, with_tri, &total);
-                ++np;
-            }
-        }
-        char *dv = (char *)g_sbuf.dev;
-        rc = bxh_memcpy_h2d_async(dv, g_sbuf.host, need, st);
-        if (!rc)
-            rc = bxh_gemm_grouped(dt, (const bxh_problem_t *)dv, np,
-                                  (const bxh_seg_t *)(dv + prob_bytes), total, 0, st);
-        if (!rc) rc = bxh_event_record(g_sbuf.done, st);
-        if (!rc) {
-            BX_STAT_ADD(kernel_launches, 1);
-            bx_stat_flops(nseg * (dt == BLASX_Z ? 4.0 : 1.0) * (double)N * (N + 1) * K);
-        }
+        BX_STAT_ADD(kernel_launches, 1);
+        bx_stat_flops(P.nseg * (dt == BLASX_Z ? 4.0 : 1.0) * (double)N * (N + 1) * K);
     }
-    pthread_mutex_unlock(&g_slock);
     return rc;
 }
 

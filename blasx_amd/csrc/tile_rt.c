@@ -36,6 +36,7 @@
 #include <string.h>
 
 #include "internal.h"
+#include "tilecost.h"
 
 #define BX_SLOT_BYTES ((size_t)2048 * 2048 * 8) /* one FP64 2048^2 tile: 32 MiB */
 #define BX_CHUNK_BYTES ((size_t)1 << 30)
@@ -363,11 +364,41 @@ static void choose_round_shape(plan_t *p, int cap_slots)
     p->RN = RN;
 }
 
+/* The block tile shape of a round's C tiles (cache slots are 16-byte aligned,
+ * so every operand takes the DMA): the one whose tiles, shared out over 256
+ * CUs, take the least time (tilecost.h).  Tile counts and starts on it; the
+ * launch's grid argument in *grid. */
+static int round_tiles(int dt, bxh_problem_t *prob, int n, int64_t K, int *grid)
+{
+    static const int shape[BXC_SHAPES] = {BXH_SHAPE_32x32, -1, BXH_SHAPE_64x64, BXH_SHAPE_128x64,
+                                          BXH_SHAPE_128x128};
+    int best = BXC_64x64, total = 0;
+    double bt = 1e300;
+    for (int s = 0; s < BXC_SHAPES; ++s) {
+        const bx_cost_t *c = &BX_COST_DMA[dt][s];
+        if (shape[s] < 0 || c->a <= 0) continue;
+        int64_t tiles = 0;
+        for (int i = 0; i < n; ++i) tiles += bx_cost_tiles(s, prob[i].m, prob[i].n);
+        const double t = c->l + (double)((tiles + 255) / 256) * bx_cost_tile(c, K);
+        if (t < bt) bt = t, best = s;
+    }
+    for (int i = 0; i < n; ++i) {
+        bxh_problem_t *P = &prob[i];
+        P->shape = shape[best];
+        P->form = BXH_FORM_DMA;
+        P->tiles_m = (P->m + BX_COST_BM[best] - 1) / BX_COST_BM[best];
+        P->tiles_n = (P->n + BX_COST_BN[best] - 1) / BX_COST_BN[best];
+        P->tile_start = total;
+        total += P->tiles_m * P->tiles_n;
+    }
+    *grid = best >= BXC_128x64 ? BXH_GROUP_BIG : 0;
+    return total;
+}
+
 static int run_plan(plan_t *p, bx_cache_t *c)
 {
     const int es = p->es, T = p->T;
     const int R = p->RM * p->RN;
-    const int bm = bxh_tile_m(p->dt), bn = bxh_tile_n(p->dt);
     const size_t prob_bytes = (size_t)R * sizeof(bxh_problem_t);
     const size_t seg_off_bytes = (prob_bytes + 255) & ~(size_t)255;
     const size_t desc_bytes = seg_off_bytes + (size_t)R * p->kt * sizeof(bxh_seg_t);
@@ -448,7 +479,6 @@ static int run_plan(plan_t *p, bx_cache_t *c)
         bxh_seg_t *seg = (bxh_seg_t *)(desc + seg_off_bytes);
 
         /* C tiles in, problem descriptors */
-        int tiles_total = 0;
         for (int t = 0; t < ntile; ++t) {
             const int ii = tii[t], kk = tkk[t];
             const int i = i0 + ii, k = k0 + kk;
@@ -476,10 +506,6 @@ static int run_plan(plan_t *p, bx_cache_t *c)
             P->seg_off = t * p->kt;
             P->opa = p->opa;
             P->opb = p->opb;
-            P->tiles_m = (mc + bm - 1) / bm;
-            P->tiles_n = (nc + bn - 1) / bn;
-            P->tile_start = tiles_total;
-            tiles_total += P->tiles_m * P->tiles_n;
             P->beta_zero = p->beta_zero;
             P->alpha_re = p->alpha[0];
             P->alpha_im = p->alpha[1];
@@ -561,6 +587,8 @@ static int run_plan(plan_t *p, bx_cache_t *c)
 
         /* compute after this round's copies; descriptors ride the compute stream */
         const int nprob = ntile;
+        int grid;
+        const int tiles_total = round_tiles(p->dt, prob, nprob, p->K, &grid);
         if ((rc = bxh_event_record(g_rt.ev_h2d[d], g_bx.s_h2d))) break;
         if ((rc = bxh_stream_wait_event(g_bx.s_comp, g_rt.ev_h2d[d]))) break;
         if ((rc = bxh_memcpy_h2d_async(g_rt.desc_dev[d], g_rt.desc_host[d],
@@ -569,7 +597,7 @@ static int run_plan(plan_t *p, bx_cache_t *c)
             break;
         char *ddev = (char *)g_rt.desc_dev[d];
         if ((rc = bxh_gemm_grouped(p->dt, (const bxh_problem_t *)ddev, nprob,
-                                   (const bxh_seg_t *)(ddev + seg_off_bytes), tiles_total, 0,
+                                   (const bxh_seg_t *)(ddev + seg_off_bytes), tiles_total, grid,
                                    g_bx.s_comp)))
             break;
         BX_STAT_ADD(kernel_launches, 1);
