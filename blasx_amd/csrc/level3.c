@@ -414,14 +414,21 @@ static int gpu_trsm(int dt, int side, int uplo, int trans, int diag, int M, int 
     void *dA, *dT, *dB, *dX;
     int64_t lB;
     pthread_mutex_lock(&g_bx.gpu_lock);
-    /* T = op(A), dense and triangular (lower when lowerT) */
-    int rc = dev_copy(&s, A, na, lda, es, &dA);
+    /* T = op(A), triangular (lower when lowerT): A itself where it is in HBM
+     * and nothing has to be written to it, else a dense copy */
+    int rc = 0;
+    int64_t lT = na;
+    if (bx_in_hbm(A) && (trans != CblasNoTrans || diag == CblasNonUnit))
+        dA = (void *)A, lT = lda;
+    else
+        rc = dev_copy(&s, A, na, lda, es, &dA);
     int lowerT = uplo == CblasLower;
     dT = dA;
     if (!rc && trans != CblasNoTrans) {
         rc = scratch_alloc(&s, &dT, (size_t)na * na * es);
-        if (!rc) rc = bxh_transpose(dt, na, na, dA, na, dT, na, trans == CblasConjTrans, g_bx.s_comp);
+        if (!rc) rc = bxh_transpose(dt, na, na, dA, lT, dT, na, trans == CblasConjTrans, g_bx.s_comp);
         lowerT = !lowerT;
+        lT = na;
     }
     if (!rc && diag == CblasUnit) rc = bxh_tri_fill(dt, na, lowerT, BX_FILL_UNIT, dT, na, g_bx.s_comp);
     if (!rc) rc = dev_view(&s, B, M, N, ldb, es, 1, &dB, &lB);
@@ -433,12 +440,12 @@ static int gpu_trsm(int dt, int side, int uplo, int trans, int diag, int M, int 
     if (!rc && side == CblasLeft) {
         /* op(A) X = alpha B, solved in place */
         if (!alpha_one) rc = scale_any(dt, M, N, al, dB, lB);
-        if (!rc) rc = trsm_rec(dt, &w, lowerT, dT, na, dB, lB, M, N, es);
+        if (!rc) rc = trsm_rec(dt, &w, lowerT, dT, lT, dB, lB, M, N, es);
     } else if (!rc) {
         /* X op(A) = alpha B  <=>  op(A)^T X^T = alpha B^T: solve on B^T with T^T */
         void *dTt;
         rc = scratch_alloc(&s, &dTt, (size_t)na * na * es);
-        if (!rc) rc = bxh_transpose(dt, na, na, dT, na, dTt, na, 0, g_bx.s_comp);
+        if (!rc) rc = bxh_transpose(dt, na, na, dT, lT, dTt, na, 0, g_bx.s_comp);
         if (!rc) rc = scratch_alloc(&s, &dX, (size_t)N * M * es);
         if (!rc) rc = bxh_transpose(dt, M, N, dB, lB, dX, N, 0, g_bx.s_comp);
         if (!rc && !alpha_one) rc = scale_any(dt, N, M, al, dX, N);

@@ -256,6 +256,38 @@ def test_gpu_trsm(gpu, orc, dt, where):
                     assert err <= tol, f"trsm backward error {err:.3e} > {tol:.3e}"
 
 
+@pytest.mark.parametrize("m", [1, 5, 63, 64])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_gpu_trsm_quotients_are_divisions(gpu, dt, m):
+    """a diagonal T of one leaf: X must be B / T(k,k) as IEEE division rounds
+    it, for quotients and diagonals in and out of the exponents that the
+    reciprocal serves, zeros and subnormal results among them"""
+    bx = gpu
+    N = 20000
+    span = 900 if dt == np.float64 else 100
+    rng = np.random.default_rng(m)
+    for wide in (0, 1, 2):  # exponents: near 0; wide in B; wide in both
+        for uplo in (UP, LO):
+            say("trsm quotients", np.dtype(dt).name, m, wide, uplo)
+            e = rng.integers(-span // 2, span // 2, m) if wide == 2 else np.zeros(m, int)
+            d = np.ldexp(rng.uniform(1, 2, m), e).astype(dt)
+            B = rng.uniform(-1, 1, (m, N))
+            if wide:
+                B = np.ldexp(B, rng.integers(-span // 2 - 100 * (span > 100), span // 2, (m, N)))
+            B = B.astype(dt)
+            B[rng.random((m, N)) < 0.1] = 0
+            A = np.asfortranarray(np.diag(d))
+            dA, dB = _dev(bx, A), _dev(bx, np.asfortranarray(B))
+            call(bx.lib(), "cblas", PFX[dt] + "trsm", dt, COL, LEFT, uplo, NOTR, NONUNIT, m, N,
+                 1.0, dA.ptr, m, dB.ptr, m)
+            X = dB.download()
+            dA.free()
+            dB.free()
+            with np.errstate(all="ignore"):
+                ref = B / d[:, None]
+            assert np.array_equal(X, ref), (np.dtype(dt).name, m, wide, uplo)
+
+
 def test_gpu_trsm_exact_integers_and_row_major(gpu, orc):
     """unit triangular integer T and integer X: B = T X is exact, so the solve
     must give X back bit for bit (ragged leaves, both triangles, both sides,
