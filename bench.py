@@ -1321,7 +1321,7 @@ def main():
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3),
                      "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / FP64_PEAK_TFLOPS, 4), "traffic": traffic,
-                     "kernel": "k_dgemm_dma<MN,K> (FP64 MFMA 16x16x4, global->LDS DMA staging)",
+                     "kernel": "k_tile<double, MN, K, 128x128> (FP64 MFMA 16x16x4, global->LDS DMA staging)",
                      "launch_ms": round(avg_ms, 3)},
         "check": {"max_err_over_gammaK_bound": float(f"{check:.3e}"),
                   "passed": check < 1.0,

@@ -23,17 +23,17 @@ template <typename E> struct Cfg;
 // gfx950: the FP32 16x16x4 MFMA returns rows 4*lg + v, the FP64 16x16x4
 // MFMA returns rows lg + 4*v.
 template <> struct Cfg<double> {
-    static constexpr int BM = 128, BN = 128, BK = 16, VEC = 2, PADA = 2, PADB = 2;
+    static constexpr int BM = 128, BN = 128;
     typedef d4_t acc_t;
     static __device__ __forceinline__ int out_row(int lg, int v) { return lg + 4 * v; }
 };
 template <> struct Cfg<float> {
-    static constexpr int BM = 128, BN = 128, BK = 32, VEC = 4, PADA = 4, PADB = 4;
+    static constexpr int BM = 128, BN = 128;
     typedef f4_t acc_t;
     static __device__ __forceinline__ int out_row(int lg, int v) { return 4 * lg + v; }
 };
 template <> struct Cfg<cplx> {
-    static constexpr int BM = 128, BN = 64, BK = 8, VEC = 1, PADA = 1, PADB = 1;
+    static constexpr int BM = 128, BN = 64;
     typedef d4_t acc_t;
     static __device__ __forceinline__ int out_row(int lg, int v) { return lg + 4 * v; }
 };
@@ -43,9 +43,6 @@ enum { MAJ_MN = 0, MAJ_K = 1 };
 
 template <typename E> __device__ __forceinline__ E zero_of() { return E(0); }
 template <> __device__ __forceinline__ cplx zero_of<cplx>() { return cplx{0.0, 0.0}; }
-
-template <typename E> __device__ __forceinline__ E conj_of(E x) { return x; }
-template <> __device__ __forceinline__ cplx conj_of<cplx>(cplx x) { return cplx{x.re, -x.im}; }
 
 // The epilogue's arithmetic, one rounding sequence for every kernel (explicit
 // FMAs: no result depends on how the compiler contracts a kernel's code).

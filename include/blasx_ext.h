@@ -188,8 +188,8 @@ int blasx_dgemm_bf16x3_device(int transa, int transb, int M, int N, int K, doubl
 /* ---- grouped GEMM -----------------------------------------------------------
  * No counterpart in the reference (which issues one vendor call per tile
  * product, blas/blasx_dgemm.c:87-94).  Many independent GEMMs of mixed
- * shape, transposes and element type (S, D, Z) in one launch per element
- * type; pointers are HBM addresses.  Asynchronous on `stream`. */
+ * shape, transposes and element type (S, D, Z) in at most two launches per
+ * element type; pointers are HBM addresses.  Asynchronous on `stream`. */
 typedef struct blasx_gemm_desc {
     int dtype;              /* BLASX_S, BLASX_D or BLASX_Z */
     int transa, transb;     /* CBLAS enums (111/112/113) */
@@ -207,8 +207,9 @@ typedef struct blasx_gemm_desc {
 int blasx_gemm_grouped_device(const blasx_gemm_desc_t *descs, int n, void *stream);
 
 /* Block tile shape of a real problem in a grouped launch (or a server
- * batch): 0 = 128 x 128, 1 = 128 x 64, 2 = 64 x 64; complex problems keep
- * 128 x 64.  No counterpart in the reference (its tile sizes are compile-time
+ * batch): 0 = 128 x 128, 1 = 128 x 64, 2 = 64 x 64 (which a launch with too
+ * few tiles cuts to 32 x 32).  Complex problems, and operands without
+ * 16-byte alignment, take the nearest shape that they have.  No counterpart in the reference (its tile sizes are compile-time
  * constants, include/blasx.h:5-7).  The shape is picked per problem from a
  * table of launch times measured on an MI355X (built in, written by
  * python -m blasx_amd.tune --grouped; entries added at run time carry a
