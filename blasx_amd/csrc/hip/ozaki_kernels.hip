@@ -1238,9 +1238,7 @@ __device__ __forceinline__ void crt_tile_origin(int np, int &m0, int &n0)
     crt_tile_origin_of((int)blockIdx.x, (int)gridDim.x, np, m0, n0);
 }
 
-// product p0 + blockIdx.y.  The host launches one product at a time when
-// one fills the GPU: measured at 16384^3, a single launch over all products
-// ran the same blocks 5% slower.
+// product p0 + blockIdx.y
 __global__ __launch_bounds__(OZ_NT_BIG, 1) void k_crt_gemm_big(const OzSeg *__restrict__ segs,
                                                                int kp, int np, int per, CrtMods md,
                                                                int8_t *__restrict__ R, int64_t ldr,
@@ -1593,9 +1591,13 @@ int bxh_crt_gemm(const void *segs_dev, int L, int per, const int *moduli, int kp
                               ? (mp / OZ_BIG) * (np / OZ_BIG)
                               : 0;
     if (big_tiles * nprod >= 256) {
-        // one launch per product when one product fills the GPU, else all
-        // products in one launch
-        const int per_launch = big_tiles >= 256 ? 1 : nprod;
+        // one launch per product from 1024 tiles (four rounds of the CUs) up,
+        // else all products in one launch, whose rounds run into each other.
+        // One launch per product against one for all, DGEMM with 16 moduli:
+        // 4096^3 1339 -> 1284 us, 4608x4608x2048 1373 -> 1015, 5120^3 2617 ->
+        // 2273, 6144^3 4591 -> 3949, 8192x8192x2048 2877 -> 2795; but 8192^3
+        // 8315 -> 8380, and 5% slower at 16384^3.
+        const int per_launch = big_tiles >= 1024 ? 1 : nprod;
         for (int p = 0; p < nprod; p += per_launch)
             hipLaunchKernelGGL(k_crt_gemm_big, dim3(big_tiles, per_launch), dim3(OZ_NT_BIG), 0,
                                (hipStream_t)stream, (const OzSeg *)segs_dev, kp, np, per, md, R,

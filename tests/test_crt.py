@@ -362,6 +362,31 @@ def test_gpu_crt_exact_integers_and_beta_zero(gpu, orc):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(4096, 4096), (7936, 8448), (8192, 8192)])
+def test_gpu_crt_products_in_one_launch(gpu, M, N):
+    """256, 1023 and 1024 big tiles, about where the products move from one
+    launch to one each: an entry depends on its row and column only, so
+    blocks equal, bit for bit, what a small call (128x128 tiles) gives"""
+    bx = gpu
+    K, n = 128, 200
+    rng = np.random.default_rng(M)
+    A, B = (np.asfortranarray(rng.uniform(-1, 1, x)) for x in ((M, K), (K, N)))
+    dA, dB, dC, dR = (bx.DeviceArray.from_host(x) for x in (A, B, np.zeros((M, N), order="F"),
+                                                          np.zeros((n, n), order="F")))
+    say("crt launches", M, N, K)
+    bx.dgemm_crt_device("N", "N", M, N, K, 1.0, dA.ptr, M, dB.ptr, K, 0.0, dC.ptr, M, 16)
+    bx.synchronize()
+    out = dC.download()
+    for r0, c0 in [(0, 0), (M - n, N - n), (M // 2 - 100, 0), (0, N - n), (M - n, 1999)]:
+        bx.dgemm_crt_device("N", "N", n, n, K, 1.0, dA.ptr + 8 * r0, M, dB.ptr + 8 * c0 * K, K,
+                            0.0, dR.ptr, n, 16)
+        bx.synchronize()
+        assert np.array_equal(out[r0:r0 + n, c0:c0 + n], dR.download()), (r0, c0)
+    for d in (dA, dB, dC, dR):
+        d.free()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "T")])
 def test_gpu_crt_big_tile_path_sampled(gpu, orc, ta, tb):
     """M, N >= 4096 pads to 256 and runs the 256x256 INT8 kernel; ragged M,
