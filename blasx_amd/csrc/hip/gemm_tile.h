@@ -82,10 +82,12 @@ template <typename E, int MAJ, int ROWS> struct Stage {
 
 // 16 bytes per lane from global memory to LDS at lds + 16 lane (`lds`
 // wave-uniform).  M0 is reserved: the compiler does not allocate it, and
-// nothing else in these kernels uses it.
+// nothing else in these kernels uses it.  A load to LDS may read the old M0 in
+// the cycle after a scalar write of it: one wait state between them, which the
+// compiler does not put inside inline assembly.
 __device__ __forceinline__ void dma16_lds(const void *base, uint32_t off, uint32_t lds)
 {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :
                  : "s"(lds), "v"(off), "s"(base)
                  : "memory");

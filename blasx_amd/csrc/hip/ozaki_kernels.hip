@@ -417,10 +417,12 @@ __device__ __forceinline__ void lgkm_wait0()
 // wave's destination, a wave-uniform LDS address held in a scalar register.
 // M0 is a reserved register the compiler does not allocate (a clobber of it
 // is ignored); nothing else in the kernels that call this uses M0 (checked
-// in their gfx950 assembly: every M0 write is this statement's).
+// in their gfx950 assembly: every M0 write is this statement's).  A load to
+// LDS needs one wait state after a scalar write of M0, which the compiler does
+// not put inside inline assembly.
 __device__ __forceinline__ void dma16_at(const int8_t *g, uint32_t lds)
 {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                  :
                  : "s"(lds), "v"(g)
                  : "memory");
