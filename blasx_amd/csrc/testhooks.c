@@ -142,6 +142,19 @@ BX_EXPORT int bxtest_plan_simulate(int dt, int opa, int opb, int M, int N, int K
                             evictions, mode, nbands);
 }
 
+/* the block tile shape, movement and grid argument of a round of one C tile */
+int bx_round_tiles(int dt, int T, bxh_problem_t *prob, int n, int64_t K, int *grid);
+BX_EXPORT int bxtest_round_tile(int dt, int T, int opa, int opb, int M, int N, int K, int *shape,
+                                int *form, int *grid)
+{
+    bxh_problem_t P = {0};
+    P.m = M, P.n = N, P.opa = opa, P.opb = opb;
+    const int total = bx_round_tiles(dt, T, &P, 1, K, grid);
+    *shape = P.shape;
+    *form = P.form;
+    return total;
+}
+
 /* HER2K's unimodular factor (level3.c) */
 void bx_her2k_factor(const double *a, int conj_ratio, double *out);
 BX_EXPORT void bxtest_her2k_factor(double re, double im, int conj_ratio, double *out)

@@ -364,18 +364,25 @@ static void choose_round_shape(plan_t *p, int cap_slots)
     p->RN = RN;
 }
 
-/* The block tile shape of a round's C tiles (cache slots are 16-byte aligned,
- * so every operand takes the DMA): the one whose tiles, shared out over 256
- * CUs, take the least time (tilecost.h).  Tile counts and starts on it; the
- * launch's grid argument in *grid. */
-static int round_tiles(int dt, bxh_problem_t *prob, int n, int64_t K, int *grid)
+/* The block tile shape of a round's C tiles, T the tile edge (and leading
+ * dimension in the cache slots, whose bases are 16-byte aligned): the one
+ * whose tiles, shared out over 256 CUs, take the least time (tilecost.h).  A T
+ * whose columns are not all 16-byte aligned (a tune file may hold any) takes
+ * the small shapes, through registers.  Tile counts and starts on the shape;
+ * the launch's grid argument in *grid. */
+int bx_round_tiles(int dt, int T, bxh_problem_t *prob, int n, int64_t K, int *grid)
 {
     static const int shape[BXC_SHAPES] = {BXH_SHAPE_32x32, -1, BXH_SHAPE_64x64, BXH_SHAPE_128x64,
                                           BXH_SHAPE_128x128};
-    int best = BXC_64x64, total = 0;
+    const bxh_seg_t slot = {NULL, NULL, T, T, K};
+    int best = BXC_64x64, total = 0, dma = 1;
     double bt = 1e300;
+    for (int i = 0; i < n; ++i) {
+        prob[i].form = bxh_tile_form(dt, prob[i].opa, prob[i].opb, prob[i].m, prob[i].n, &slot);
+        if (prob[i].form != BXH_FORM_DMA) dma = 0;
+    }
     for (int s = 0; s < BXC_SHAPES; ++s) {
-        const bx_cost_t *c = &BX_COST_DMA[dt][s];
+        const bx_cost_t *c = dma ? &BX_COST_DMA[dt][s] : &BX_COST_REG[dt][s];
         if (shape[s] < 0 || c->a <= 0) continue;
         int64_t tiles = 0;
         for (int i = 0; i < n; ++i) tiles += bx_cost_tiles(s, prob[i].m, prob[i].n);
@@ -385,7 +392,6 @@ static int round_tiles(int dt, bxh_problem_t *prob, int n, int64_t K, int *grid)
     for (int i = 0; i < n; ++i) {
         bxh_problem_t *P = &prob[i];
         P->shape = shape[best];
-        P->form = BXH_FORM_DMA;
         P->tiles_m = (P->m + BX_COST_BM[best] - 1) / BX_COST_BM[best];
         P->tiles_n = (P->n + BX_COST_BN[best] - 1) / BX_COST_BN[best];
         P->tile_start = total;
@@ -588,7 +594,7 @@ static int run_plan(plan_t *p, bx_cache_t *c)
         /* compute after this round's copies; descriptors ride the compute stream */
         const int nprob = ntile;
         int grid;
-        const int tiles_total = round_tiles(p->dt, prob, nprob, p->K, &grid);
+        const int tiles_total = bx_round_tiles(p->dt, T, prob, nprob, p->K, &grid);
         if ((rc = bxh_event_record(g_rt.ev_h2d[d], g_bx.s_h2d))) break;
         if ((rc = bxh_stream_wait_event(g_bx.s_comp, g_rt.ev_h2d[d]))) break;
         if ((rc = bxh_memcpy_h2d_async(g_rt.desc_dev[d], g_rt.desc_host[d],

@@ -126,3 +126,60 @@ def test_autotuner_measures_and_records(gpu):
     assert measured[[256, 512, 1024, 2048].index(best.value)] == min(measured)
     L.blasx_get_tile_size.argtypes = [C.c_int] * 4
     assert L.blasx_get_tile_size(bx.D, 3000, 2500, 2000) == best.value
+
+
+@pytest.mark.parametrize("T", [301, 302, 303, 304, 1001, 1002, 2048])
+@pytest.mark.parametrize("dt", ["S", "D", "Z"])
+def test_round_tiles_are_moved_as_the_tile_edge_allows_cpu(bx, dt, T):
+    """A tune table may hold any tile edge, and the edge is the leading
+    dimension of the tiles in HBM: rounds move them by 16-byte DMA only where
+    every column starts on 16 bytes, else through registers on the shapes that
+    can, element by element where a column is shorter than 16 bytes."""
+    L = bx.test_lib()
+    code, es = {"S": (bx.S, 4), "D": (bx.D, 8), "Z": (bx.Z, 16)}[dt]
+    shape, form, grid = C.c_int(), C.c_int(), C.c_int()
+    for opa, opb in ((0, 0), (0, 1), (1, 0), (1, 1)):
+        for M, N in ((1, 1), (1, T), (T, 1), (T, T), (T - 1, T - 2)):
+            total = L.bxtest_round_tile(code, T, opa, opb, M, N, T, C.byref(shape), C.byref(form),
+                                        C.byref(grid))
+            case = (dt, T, opa, opb, M, N)
+            if T * es % 16 == 0:
+                assert form.value == 0, case
+            elif (not opa and M < 16 // es) or (opb and N < 16 // es):
+                assert form.value == 2, case
+            else:
+                assert form.value == 1, case
+            if form.value:  # only the 64x64 and 32x32 tiles have these movements
+                assert shape.value in (2, 3) and grid.value == 0, case
+            assert (grid.value == -1) == (shape.value in (0, 1)), case
+            bm, bn = {0: (128, 128), 1: (128, 64), 2: (64, 64), 3: (32, 32)}[shape.value]
+            assert total == -(-M // bm) * -(-N // bn), case
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,T", [(np.float64, 301), (np.float32, 301), (np.float32, 302),
+                                  (np.float64, 302)])
+def test_gpu_tile_edges_of_any_alignment(gpu, orc, dt, T):
+    """integer operands, exact in every order, through tiles of edge T"""
+    bx = gpu
+    L = bx.lib()
+    L.blasx_tune_table_add.argtypes = [C.c_int] * 5
+    M, N, K = 1203, 1105, 1010
+    code = bx.D if dt == np.float64 else bx.S
+    rng = np.random.default_rng(T)
+    try:
+        assert L.blasx_tune_table_add(code, M, N, K, T) == 0
+        for ta, tb in (("N", "N"), ("T", "T")):
+            print("[case] tile edge", T, np.dtype(dt).name, ta, tb, flush=True)
+            A, B, Cm = (bx.PinnedArray(*s, dt) for s in (
+                (M, K) if ta == "N" else (K, M), (K, N) if tb == "N" else (N, K), (M, N)))
+            for x in (A, B, Cm):
+                x.array[:] = rng.integers(-8, 9, x.array.shape)
+            ref = (3 * (A.array if ta == "N" else A.array.T).astype(np.float64) @
+                   (B.array if tb == "N" else B.array.T).astype(np.float64) - 2 * Cm.array)
+            bx.gemm(ta, tb, 3.0, A.array, B.array, -2.0, Cm.array)
+            assert np.array_equal(Cm.array, ref)
+            for x in (A, B, Cm):
+                x.free()
+    finally:  # later tests of this size take an ordinary edge again
+        L.blasx_tune_table_add(code, M, N, K, 1024)
