@@ -204,7 +204,7 @@ template <int K, int N, typename F> __device__ __forceinline__ void static_for(F
 // is RN(x/t)), which holds while nothing overflows or underflows.  A block in
 // which a diagonal or a quotient (other than zero) leaves the safe range of
 // exponents solves again with divisions.
-// 64 x 1024 block, FP64: 16.2 -> 12.0 us.
+// 64 x 1024 block, FP64: 16.2 -> 12.1 us (0.15 of them the zeros' signs).
 constexpr int LEAF_THREADS = 256;
 constexpr int LEAF_COLS = LEAF_THREADS / 4;
 
@@ -220,14 +220,16 @@ __device__ __forceinline__ bool in_range(float v)
     return e - (127 - 40) <= 80u;
 }
 
-// a / t, r = RN(1/t); bad where it may differ from the division
+// a / t, r = RN(1/t); bad where it may differ from the division.  The
+// remainder of a zero a is +0 whatever a's sign, so the correction would turn
+// -0 / t into +0 for t > 0: the result's sign is q's.
 template <typename E> __device__ __forceinline__ E quotient(E a, E t, E r, bool &bad)
 {
     if constexpr (is_cx<E>::value) return divide(a, t);
     else {
         const E q = a * r;
         bad |= q == E(0) && a != E(0);
-        return fma(fma(-q, t, a), r, q);
+        return copysign(fma(fma(-q, t, a), r, q), q);
     }
 }
 template <typename E> __device__ __forceinline__ bool unsafe(E v)

@@ -288,6 +288,39 @@ def test_gpu_trsm_quotients_are_divisions(gpu, dt, m):
             assert np.array_equal(X, ref), (np.dtype(dt).name, m, wide, uplo)
 
 
+@pytest.mark.parametrize("m", [1, 5, 64])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_gpu_trsm_zero_quotients_keep_their_sign(gpu, dt, m):
+    """zeros of either sign over diagonals of either sign: bit for bit what
+    substitution with divisions gives (the other products are exact zeros),
+    also in a block that an entry near the overflow threshold sends to them"""
+    bx = gpu
+    N = 20000  # on the GPU, not the CPU BLAS
+    rng = np.random.default_rng(m)
+    d = (rng.uniform(1, 2, m) * np.where(rng.random(m) < 0.5, -1, 1)).astype(dt)
+    B = rng.uniform(-1, 1, (m, N)).astype(dt)
+    u = rng.random((m, N))
+    B[u < 0.4], B[u < 0.2] = 0.0, -0.0
+    for uplo in (UP, LO):
+        for big in (False, True):
+            say("trsm zeros", np.dtype(dt).name, m, uplo, big)
+            B2 = B.copy()
+            if big:
+                B2[0, ::64] = np.finfo(dt).max / 8  # one column in each block
+            ref, T = B2.copy(), np.diag(d)
+            for k in range(m) if uplo == LO else range(m - 1, -1, -1):
+                ref[k] /= d[k]
+                for i in range(k + 1, m) if uplo == LO else range(k):
+                    ref[i] -= T[i, k] * ref[k]
+            dA, dB = _dev(bx, np.asfortranarray(T)), _dev(bx, np.asfortranarray(B2))
+            call(bx.lib(), "cblas", PFX[dt] + "trsm", dt, COL, LEFT, uplo, NOTR, NONUNIT, m, N,
+                 1.0, dA.ptr, m, dB.ptr, m)
+            X = dB.download()
+            dA.free()
+            dB.free()
+            assert np.array_equal(X, ref) and np.array_equal(np.signbit(X), np.signbit(ref))
+
+
 def test_gpu_trsm_exact_integers_and_row_major(gpu, orc):
     """unit triangular integer T and integer X: B = T X is exact, so the solve
     must give X back bit for bit (ragged leaves, both triangles, both sides,
