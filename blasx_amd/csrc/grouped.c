@@ -115,12 +115,29 @@ static int place_tiles(int dtype, bxh_problem_t *probs, int n)
     return total;
 }
 
+/* A complex problem's shape in a launch of `load` 128x64 tiles of its type:
+ * 128x64 where they take one round of two tiles on each of 256 CUs, while 64x64
+ * tiles, three on a CU, would begin a second, uneven one (one 2048^3 934 against
+ * 1134 us, four of 1024^3 478 against 521, 256 of 128^3 92 against 105), and no
+ * half of a tile stays empty.  With fewer tiles 64x64 or 32x32 spread better (8
+ * of 512^3: 130 against 138 us); with more the two are level on whole tiles (four
+ * of 4096^3 28.6 ms) and 64x64 ahead on ragged ones (12 of 450x1100x900 721
+ * against 842 us, 24 of 300x3000x700 1844 against 2252), until K is so long that
+ * the smaller tiles miss L2 (64 of 256x16384x8192 230 against 242 ms, two of 8192^3
+ * 114.8 against 117.0, 32 of 256x8192x4096 28.8 against 29.4). */
+static int complex_shape(int M, int K, int64_t load)
+{
+    const int over = (M + 127) / 128 * 128 - (M + 63) / 64 * 64;
+    const int one_round = load > 384 && load <= 512, long_k = load >= 2048 && K >= 4096;
+    return (one_round || long_k) && 16 * over <= M ? BXH_SHAPE_128x64 : BXH_SHAPE_64x64;
+}
+
 /* Fill problem/segment tables for the descriptors of one dtype (device
  * pointers in the descriptors).  Descriptors with alpha == 0 or K == 0 are
- * skipped (the caller scales C separately).  Each real problem's shape comes
- * from bx_grouped_shape, given the launch's load: its tile count at the large
- * tile; problems on 64x64 tiles, complex ones and those whose operands do
- * not take the DMA share one choice of 64x64 or 32x32.  The first nprob[0]
+ * skipped (the caller scales C separately).  A real problem's shape comes from
+ * bx_grouped_shape, a complex one's from complex_shape, given the launch's
+ * load: its tile count at the large tile; problems on 64x64 tiles and those
+ * whose operands do not take the DMA share one choice of 64x64 or 32x32.  The first nprob[0]
  * problems (total[0] tiles) are those, the next nprob[1] (total[1] tiles, a
  * launch of their own) the 128-row shapes; big = 0 puts all in the first. */
 void bx_grouped_fill(const blasx_gemm_desc_t *d, int n, int dtype, bxh_problem_t *probs,
@@ -141,7 +158,8 @@ void bx_grouped_fill(const blasx_gemm_desc_t *d, int n, int dtype, bxh_problem_t
         if (!desc_runs(x, dtype)) continue;
         bxh_problem_t *P = &probs[np];
         if (x->M != lm || x->N != ln || x->K != lk) {
-            shape = bx_grouped_shape(dtype, x->M, x->N, x->K, load);
+            shape = dtype == BLASX_Z ? complex_shape(x->M, x->K, load)
+                                     : bx_grouped_shape(dtype, x->M, x->N, x->K, load);
             lm = x->M;
             ln = x->N;
             lk = x->K;
@@ -165,7 +183,7 @@ void bx_grouped_fill(const blasx_gemm_desc_t *d, int n, int dtype, bxh_problem_t
         segs[np].ldb = x->ldb;
         segs[np].k = x->K;
         P->form = bxh_tile_form(dtype, P->opa, P->opb, P->m, P->n, &segs[np]);
-        P->shape = big && dtype != BLASX_Z && P->form == BXH_FORM_DMA ? shape : BXH_SHAPE_64x64;
+        P->shape = big && P->form == BXH_FORM_DMA ? shape : BXH_SHAPE_64x64;
         /* small problems stay in front of the big ones */
         if (P->shape != BXH_SHAPE_64x64)
             ++nbig;

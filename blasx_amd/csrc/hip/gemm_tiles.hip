@@ -112,33 +112,39 @@ int best_shape(int dtype, bool dma, int tri, int m, int n, int64_t k)
     return best;
 }
 
-template <typename E> void launch_tile(int s, const bxh_problem_t &P, const bxh_seg_t *S, hipStream_t st)
+// false: no such tile for this type and form
+template <typename E>
+bool launch_tile(int s, const bxh_problem_t &P, const bxh_seg_t *S, hipStream_t st)
 {
     if (P.form != BXH_FORM_DMA) {
         switch (s) {
-        case BXC_32x32: launch_shape<E, 16, 16, 2, false, 4>(P, S, st); return;
-        case BXC_64x32: launch_shape<E, 32, 16, 2, false, 4>(P, S, st); return;
-        default: launch_shape<E, 32, 32, 2, false, 3>(P, S, st); return;
+        case BXC_32x32: launch_shape<E, 16, 16, 2, false, 4>(P, S, st); return true;
+        case BXC_64x32: launch_shape<E, 32, 16, 2, false, 4>(P, S, st); return true;
+        case BXC_64x64: launch_shape<E, 32, 32, 2, false, 3>(P, S, st); return true;
         }
+        return false;
     }
     switch (s) {
-    case BXC_32x32: launch_shape<E, 16, 16, 4, true, 4>(P, S, st); return;
-    case BXC_64x32: launch_shape<E, 32, 16, 4, true, 3>(P, S, st); return;
-    case BXC_64x64: launch_shape<E, 32, 32, 4, true, 2>(P, S, st); return;
+    case BXC_32x32: launch_shape<E, 16, 16, 4, true, 4>(P, S, st); return true;
+    case BXC_64x32: launch_shape<E, 32, 16, 4, true, 3>(P, S, st); return true;
+    case BXC_64x64: launch_shape<E, 32, 32, 4, true, 2>(P, S, st); return true;
+    case BXC_128x64:
+        launch_shape<E, 64, 32, sizeof(E) == 16 ? 2 : 3, true, 2>(P, S, st);
+        return true;
     }
-    if constexpr (sizeof(E) == 16) {
-        launch_shape<E, 64, 32, 2, true, 2>(P, S, st);
-    } else {
-        if (s == BXC_128x64) launch_shape<E, 64, 32, 3, true, 2>(P, S, st);
-        else launch_shape<E, 64, 64, 2, true, 2>(P, S, st);
-    }
+    if constexpr (sizeof(E) != 16)
+        if (s == BXC_128x128) {
+            launch_shape<E, 64, 64, 2, true, 2>(P, S, st);
+            return true;
+        }
+    return false;
 }
 
 } // namespace
 
 extern "C" {
 
-int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *stream)
+int bxh_gemm_tile_as(int dtype, int shape, const bxh_problem_t *P, const bxh_seg_t *S, void *stream)
 {
     if (dtype < 0 || dtype > 2 || P->nseg < 1 || P->nseg > 2 || (P->tri && P->m != P->n))
         return BLASX_EINVAL;
@@ -151,14 +157,24 @@ int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *s
         k += S[i].k;
     }
     hipStream_t st = (hipStream_t)stream;
-    const int s = best_shape(dtype, Q.form == BXH_FORM_DMA, P->tri, P->m, P->n, k);
-    switch (dtype) {
-    case BLASX_S: launch_tile<float>(s, Q, S, st); break;
-    case BLASX_D: launch_tile<double>(s, Q, S, st); break;
-    case BLASX_Z: launch_tile<cplx>(s, Q, S, st); break;
-    default: return BLASX_EINVAL;
-    }
+    const int s =
+        shape >= 0 ? shape : best_shape(dtype, Q.form == BXH_FORM_DMA, P->tri, P->m, P->n, k);
+    const bool ran = dtype == BLASX_S   ? launch_tile<float>(s, Q, S, st)
+                     : dtype == BLASX_D ? launch_tile<double>(s, Q, S, st)
+                                        : launch_tile<cplx>(s, Q, S, st);
+    if (!ran) return BLASX_EINVAL;
     return hipGetLastError() == hipSuccess ? 0 : BLASX_EHIP;
+}
+
+int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *stream)
+{
+    return bxh_gemm_tile_as(dtype, -1, P, S, stream);
+}
+
+// the shape (BXC_*) that bxh_gemm_tile takes; for the test-suite
+int bxh_tile_shape_host(int dtype, int dma, int tri, int m, int n, int64_t k)
+{
+    return best_shape(dtype, dma != 0, tri, m, n, k);
 }
 
 } // extern "C"

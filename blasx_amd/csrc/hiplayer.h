@@ -134,10 +134,13 @@ static inline int bxh_tile_form(int dtype, int opa, int opb, int m, int n, const
  * stored triangle (tri, m == n), on the block tile shape that runs it fastest
  * (hip/gemm_tiles.hip); its form, shape and tile fields are not read */
 int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *stream);
+/* on the given shape (BXC_*, tilecost.h); BLASX_EINVAL where the type and form
+ * of the operands have no such tile */
+int bxh_gemm_tile_as(int dtype, int shape, const bxh_problem_t *P, const bxh_seg_t *S, void *stream);
 /* grouped launch over a device-resident problem and segment table; all
  * problems share dtype.  grid = 0: one block per tile, every problem's shape
  * BXH_SHAPE_64x64 or BXH_SHAPE_32x32; grid = BXH_GROUP_BIG: one block per
- * tile, every problem real, moved by DMA, of a 128-row shape. */
+ * tile, every problem moved by DMA and of a 128-row shape (complex: 128x64). */
 #define BXH_GROUP_BIG (-1)
 int bxh_gemm_grouped(int dtype, const bxh_problem_t *probs_dev, int nprob,
                      const bxh_seg_t *segs_dev, int total_tiles, int grid, void *stream);

@@ -155,6 +155,49 @@ BX_EXPORT int bxtest_round_tile(int dt, int T, int opa, int opb, int M, int N, i
     return total;
 }
 
+/* the plain GEMM and rank-k launch on a given block tile shape (BXC_*; -1:
+ * the one the library takes); B2 non-NULL: a second K segment, B2 op(A)^T;
+ * and the shape the library takes */
+BX_EXPORT int bxtest_gemm_tile(int dt, int shape, int tri, int opa, int opb, int m, int n, int k,
+                               const double *alpha, const void *A, int64_t lda, const void *B,
+                               int64_t ldb, const void *B2, int64_t ldb2, const double *beta,
+                               void *C, int64_t ldc)
+{
+    bxh_problem_t P = {0};
+    P.C = C;
+    P.ldc = ldc;
+    P.m = m, P.n = n;
+    P.nseg = B2 ? 2 : 1;
+    P.opa = opa, P.opb = opb;
+    P.tri = tri;
+    P.alpha_re = alpha[0], P.alpha_im = alpha[1];
+    P.beta_re = beta[0], P.beta_im = beta[1];
+    P.beta_zero = beta[0] == 0.0 && beta[1] == 0.0;
+    const bxh_seg_t S[2] = {{A, B, lda, ldb, k}, {B2, A, ldb2, lda, k}};
+    return bxh_gemm_tile_as(dt, shape, &P, S, NULL);
+}
+int bxh_tile_shape_host(int dtype, int dma, int tri, int m, int n, int64_t k);
+BX_EXPORT int bxtest_tile_shape(int dt, int dma, int tri, int m, int n, int64_t k)
+{
+    return bxh_tile_shape_host(dt, dma, tri, m, n, k);
+}
+
+/* the shapes of one type's problems in a grouped launch, in table order (the
+ * 128-row shapes last); the number of problems */
+BX_EXPORT int bxtest_grouped_shapes(const blasx_gemm_desc_t *d, int n, int dtype, int big,
+                                    int *shapes, int nprob[2], int total[2])
+{
+    bxh_problem_t *P = (bxh_problem_t *)calloc(n, sizeof *P);
+    bxh_seg_t *S = (bxh_seg_t *)calloc(n, sizeof *S);
+    if (!P || !S) abort();
+    bx_grouped_fill(d, n, dtype, P, S, big, nprob, total);
+    const int np = nprob[0] + nprob[1];
+    for (int i = 0; i < np; ++i) shapes[i] = P[i].shape;
+    free(P);
+    free(S);
+    return np;
+}
+
 /* HER2K's unimodular factor (level3.c) */
 void bx_her2k_factor(const double *a, int conj_ratio, double *out);
 BX_EXPORT void bxtest_her2k_factor(double re, double im, int conj_ratio, double *out)

@@ -386,7 +386,8 @@ int bx_round_tiles(int dt, int T, bxh_problem_t *prob, int n, int64_t K, int *gr
         if (shape[s] < 0 || c->a <= 0) continue;
         int64_t tiles = 0;
         for (int i = 0; i < n; ++i) tiles += bx_cost_tiles(s, prob[i].m, prob[i].n);
-        const double t = c->l + (double)((tiles + 255) / 256) * bx_cost_tile(c, K);
+        const int64_t busiest = s < BXC_128x64 ? bx_cost_group_busiest(tiles) : (tiles + 255) / 256;
+        const double t = c->l + (double)busiest * bx_cost_tile(c, K);
         if (t < bt) bt = t, best = s;
     }
     for (int i = 0; i < n; ++i) {
