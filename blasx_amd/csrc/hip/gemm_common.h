@@ -8,6 +8,10 @@
 #include "blasx_ext.h"
 #include "gmem.h"
 
+// 0, or BLASX_EHIP with the launch's own error kept for bxh_last_error
+// (gemm_kernels.hip)
+extern "C" int bx_launch_status(const char *what);
+
 namespace {
 
 typedef double d4_t __attribute__((ext_vector_type(4)));

@@ -127,7 +127,7 @@ int launch_group(const bxh_problem_t *probs, int nprob, const bxh_seg_t *segs, i
         if (grid <= 0 || (!counts && grid > total)) grid = total;
         hipLaunchKernelGGL(k_group<E>, dim3(grid), dim3(NT), 0, st, probs, nprob, segs, total, counts);
     }
-    return hipGetLastError() == hipSuccess ? 0 : BLASX_EHIP;
+    return bx_launch_status("grouped gemm launch");
 }
 
 } // namespace

@@ -192,6 +192,13 @@ extern "C" {
 
 const char *bxh_kernel_error(void) { return g_err; }
 
+// the outcome of the kernel launch before it
+int bx_launch_status(const char *what)
+{
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : fail(what, e);
+}
+
 void bxh_tile_dims(int dtype, int shape, int *bm, int *bn)
 {
     switch (shape) {
@@ -255,21 +262,18 @@ int bxh_gemm(int dtype, int opa, int opb, int m, int n, int k, const double *alp
         const int r = dgemm_repacked(opa != 0, opb != 0, P, S, st);
         if (r) return r < 0 ? r : 0;
     }
-    const int rc = bxh_gemm_tile(dtype, &P, &S, st);
-    return rc ? fail("gemm launch", hipErrorLaunchFailure) : 0;
+    return bxh_gemm_tile(dtype, &P, &S, st);
 }
 
 static int launch_grouped(int dtype, const bxh_problem_t *probs, int nprob, const bxh_seg_t *segs,
                           int total, int grid, const int *counts, void *stream)
 {
-    int rc;
     switch (dtype) {
-    case BLASX_S: rc = bx_launch_group_s(probs, nprob, segs, total, grid, counts, stream); break;
-    case BLASX_D: rc = bx_launch_group_d(probs, nprob, segs, total, grid, counts, stream); break;
-    case BLASX_Z: rc = bx_launch_group_z(probs, nprob, segs, total, grid, counts, stream); break;
-    default: return BLASX_EINVAL;
+    case BLASX_S: return bx_launch_group_s(probs, nprob, segs, total, grid, counts, stream);
+    case BLASX_D: return bx_launch_group_d(probs, nprob, segs, total, grid, counts, stream);
+    case BLASX_Z: return bx_launch_group_z(probs, nprob, segs, total, grid, counts, stream);
     }
-    return rc == BLASX_EHIP ? fail("grouped gemm launch", hipErrorLaunchFailure) : rc;
+    return BLASX_EINVAL;
 }
 
 int bxh_gemm_grouped(int dtype, const bxh_problem_t *probs_dev, int nprob,

@@ -163,7 +163,7 @@ int bxh_gemm_tile_as(int dtype, int shape, const bxh_problem_t *P, const bxh_seg
                      : dtype == BLASX_D ? launch_tile<double>(s, Q, S, st)
                                         : launch_tile<cplx>(s, Q, S, st);
     if (!ran) return BLASX_EINVAL;
-    return hipGetLastError() == hipSuccess ? 0 : BLASX_EHIP;
+    return bx_launch_status(P->tri ? "rank-k launch" : "gemm launch");
 }
 
 int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *stream)

@@ -176,6 +176,14 @@ BX_EXPORT int bxtest_gemm_tile(int dt, int shape, int tri, int opa, int opb, int
     const bxh_seg_t S[2] = {{A, B, lda, ldb, k}, {B2, A, ldb2, lda, k}};
     return bxh_gemm_tile_as(dt, shape, &P, S, NULL);
 }
+BX_EXPORT const char *bxtest_last_error(void) { return bxh_last_error(); }
+/* a grouped launch without a GPU (its tables are never read) */
+BX_EXPORT int bxtest_gemm_grouped(int dt, int grid)
+{
+    static bxh_problem_t P;
+    static bxh_seg_t S;
+    return bxh_gemm_grouped(dt, &P, 1, &S, 1, grid, NULL);
+}
 int bxh_tile_shape_host(int dtype, int dma, int tri, int m, int n, int64_t k);
 BX_EXPORT int bxtest_tile_shape(int dt, int dma, int tri, int m, int n, int64_t k)
 {
