@@ -281,8 +281,9 @@ BX_EXPORT int blasx_gemm_grouped_device(const blasx_gemm_desc_t *d, int n, void 
         for (int k = 0; k < 3; ++k) {
             first[k] = used;
             bx_grouped_fill(d, n, dts[k], probs + used, segs + used, 1, np[k], total[k]);
-            used += np[k][0] + np[k][1];
-            flops += desc_flops(d, n, dts[k]);
+            const int runs = np[k][0] + np[k][1];
+            used += runs;
+            if (runs) flops += desc_flops(d, n, dts[k]);
         }
         if (used) rc = bxh_memcpy_h2d_async(g_gring[slot].dev, g_gring[slot].host, need, st);
     }

@@ -90,6 +90,25 @@ def test_grouped_uneven_mixed(gpu, orc):
         assert np.array_equal(solo.download(), out)
 
 
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_grouped_work_counted_is_the_products(gpu, orc, noalloc):
+    """a type whose problems are all scaled only (alpha = 0 or K = 0) adds no
+    FLOPs to the statistics"""
+    bx = gpu
+    p = _fixed(orc, np.float32, "N", "N", 64, 64, 64, 3, alpha=0.0)
+    q = _fixed(orc, np.float64, "N", "N", 64, 96, 32, 4)
+    dev = [[bx.DeviceArray.from_host(x[k]) for k in ("A", "B", "C0")] for x in (p, q)]
+    descs = [bx.make_desc(x["dt"], "N", "N", x["M"], x["N"], x["K"], x["alpha"], d[0].ptr, x["M"],
+                          d[1].ptr, x["K"], x["beta"], d[2].ptr, x["M"])
+             for x, d in zip((p, q), dev)]
+    say("grouped work counted", noalloc)
+    for used, want in ((descs[:1], 0.0), (descs, 2.0 * 64 * 96 * 32)):
+        bx.reset_stats()
+        bx.gemm_grouped_device(used, noalloc=noalloc)
+        bx.synchronize()
+        assert bx.stats()["flops"] == want
+
+
 def _fixed(orc, dt, ta, tb, M, N, K, seed, alpha=1.25, beta=-0.5):
     A = orc.fill_uniform(M if ta == "N" else K, K if ta == "N" else M, seed, 0, dtype=dt)
     B = orc.fill_uniform(K if tb == "N" else N, N if tb == "N" else K, seed, 1, dtype=dt)
