@@ -103,10 +103,11 @@ __host__ __device__ __forceinline__ void striped(int64_t loc, int rows, int cols
     }
 }
 template <int G>
-__device__ __forceinline__ void tile_coords_striped(int t, int tiles_m, int tiles_n, int &tm, int &tn)
+__host__ __device__ __forceinline__ void tile_coords_striped(int t, int tiles_m, int tiles_n, int &tm,
+                                                             int &tn)
 {
     const int64_t per = (int64_t)G * tiles_n;
-    const int g = (int)(t / per), rows = min(tiles_m - g * G, G);
+    const int g = (int)(t / per), rows = tiles_m - g * G < G ? tiles_m - g * G : G;
     int r;
     striped(t - g * per, rows, tiles_n, r, tn);
     tm = g * G + r;

@@ -4,8 +4,8 @@
 // NEG modifier).  The reference hands the same product to cuBLAS
 // (blas/blasx_dgemm.c:87-94, blas/blasx_sgemm.c:87, blas/blasx_zgemm.c:88).
 //
-// 256 threads, 2x2 waves of WTM x WTN, four block shapes: 32x32, 64x32, 64x64
-// and 128x64.  What bounds a tile is the matrix core's issue: one FP64 MFMA
+// 256 threads, 2x2 waves of WTM x WTN, five block shapes: 32x32, 64x32, 64x64,
+// 128x64 and 128x128 (FP64, and FP32 in grouped launches).  What bounds a tile is the matrix core's issue: one FP64 MFMA
 // takes 64 cycles of its SIMD (FP32: 32), back to back even in one dependent
 // chain, and every vector ALU instruction beside it takes its slot.  So the K
 // loop has none: operand addresses are scalar bases plus constant lane

@@ -132,7 +132,7 @@ bool launch_tile(int s, const bxh_problem_t &P, const bxh_seg_t *S, hipStream_t 
         launch_shape<E, 64, 32, sizeof(E) == 16 ? 2 : 3, true, 2>(P, S, st);
         return true;
     }
-    if constexpr (sizeof(E) != 16)
+    if constexpr (sizeof(E) == 8)
         if (s == BXC_128x128) {
             launch_shape<E, 64, 64, 2, true, 2>(P, S, st);
             return true;
@@ -171,7 +171,28 @@ int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *s
     return bxh_gemm_tile_as(dtype, -1, P, S, stream);
 }
 
-// the shape (BXC_*) that bxh_gemm_tile takes; for the test-suite
+// for the test-suite: the tile of block t of a launch of a shape's tiles (tri:
+// BX_TRI_* bits, the triangular walk; else the striped one), false past the
+// grid; and the shape (BXC_*) that bxh_gemm_tile takes
+int bxh_tile_at_host(int shape, int tri, int m, int n, int64_t t, int *tm, int *tn)
+{
+    const int tiles_m = (m + BX_COST_BM[shape] - 1) / BX_COST_BM[shape];
+    const int tiles_n = (n + BX_COST_BN[shape] - 1) / BX_COST_BN[shape];
+    if (t >= shape_tiles(shape, tri, m, n)) return 0;
+    if (!tri) {
+        tile_coords_striped<G_BIG>((int)t, tiles_m, tiles_n, *tm, *tn);
+        return 1;
+    }
+    const int up = tri & BX_TRI_UPPER;
+    switch (shape) {
+    case BXC_32x32: tri_coords<G_TRI, 32, 32>(t, up, tiles_m, tiles_n, *tm, *tn); break;
+    case BXC_64x32: tri_coords<G_TRI, 64, 32>(t, up, tiles_m, tiles_n, *tm, *tn); break;
+    case BXC_64x64: tri_coords<G_TRI, 64, 64>(t, up, tiles_m, tiles_n, *tm, *tn); break;
+    case BXC_128x64: tri_coords<G_TRI, 128, 64>(t, up, tiles_m, tiles_n, *tm, *tn); break;
+    default: tri_coords<G_TRI, 128, 128>(t, up, tiles_m, tiles_n, *tm, *tn);
+    }
+    return 1;
+}
 int bxh_tile_shape_host(int dtype, int dma, int tri, int m, int n, int64_t k)
 {
     return best_shape(dtype, dma != 0, tri, m, n, k);

@@ -176,6 +176,19 @@ BX_EXPORT int bxtest_gemm_tile(int dt, int shape, int tri, int opa, int opb, int
     const bxh_seg_t S[2] = {{A, B, lda, ldb, k}, {B2, A, ldb2, lda, k}};
     return bxh_gemm_tile_as(dt, shape, &P, S, NULL);
 }
+int bxh_tile_at_host(int shape, int tri, int m, int n, int64_t t, int *tm, int *tn);
+/* the tiles of every block of a launch into tiles[2 t]; how many (-1: more than cap) */
+BX_EXPORT int64_t bxtest_tile_walk(int shape, int tri, int m, int n, int *tiles, int64_t cap)
+{
+    int tm, tn;
+    int64_t t = 0;
+    for (; bxh_tile_at_host(shape, tri, m, n, t, &tm, &tn); ++t) {
+        if (t == cap) return -1;
+        tiles[2 * t] = tm;
+        tiles[2 * t + 1] = tn;
+    }
+    return t;
+}
 BX_EXPORT const char *bxtest_last_error(void) { return bxh_last_error(); }
 /* a grouped launch without a GPU (its tables are never read) */
 BX_EXPORT int bxtest_gemm_grouped(int dt, int grid)

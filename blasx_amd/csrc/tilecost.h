@@ -29,14 +29,14 @@
 enum { BXC_32x32, BXC_64x32, BXC_64x64, BXC_128x64, BXC_128x128, BXC_SHAPES };
 
 typedef struct {
-    float l, c, a; /* a <= 0: no such tile */
+    float l, c, a; /* a <= 0: no such tile, or (FP32 128x128) never a better one */
 } bx_cost_t;
 
 static const int BX_COST_BM[BXC_SHAPES] = {32, 64, 64, 128, 128};
 static const int BX_COST_BN[BXC_SHAPES] = {32, 32, 64, 64, 128};
 /* by element type (S, D, Z): operands by DMA, and through registers */
 static const bx_cost_t BX_COST_DMA[3][BXC_SHAPES] = {
-    {{3.0f, 0.53f, 3.99f}, {3.4f, 0.88f, 7.39f}, {3.8f, 1.71f, 14.9f}, {5.7f, 4.5f, 29.3f}, {5.7f, 9.0f, 58.6f}},
+    {{3.0f, 0.53f, 3.99f}, {3.4f, 0.88f, 7.39f}, {3.8f, 1.71f, 14.9f}, {5.7f, 4.5f, 29.3f}, {0, 0, 0}},
     {{2.5f, 0.56f, 7.75f}, {3.0f, 0.87f, 14.39f}, {3.7f, 1.69f, 28.4f}, {5.6f, 2.19f, 56.6f}, {5.6f, 9.0f, 112.6f}},
     {{0.5f, 0.75f, 30.2f}, {8.2f, 0.80f, 56.8f}, {10.5f, 2.45f, 111.1f}, {130.0f, 2.2f, 214.0f}, {0, 0, 0}},
 };

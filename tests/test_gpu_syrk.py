@@ -2,7 +2,7 @@
 f77 forms) against the oracle's naive GEMM with B = A on the stored
 triangle.  The reference computes these on the CPU BLAS (blas/dsyrk.c:46-58);
 here host operands run on the tile runtime (C tiles of the triangle only,
-diagonal tiles masked) and HBM operands as one grouped launch.
+diagonal tiles masked) and HBM operands as one triangular launch.
 
 Tolerance: ||C_gpu - C_ref||_F / (|alpha| ||A||_F^2 + |beta| ||C0||_F) <= c K eps
 on the stored triangle, c = 1 real, 2 complex.  The other triangle must come

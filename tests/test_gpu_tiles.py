@@ -6,6 +6,7 @@ remainder of K, and for each way the operands are moved: 16-byte aligned,
 element aligned (odd leading dimension, offset base), and with fewer rows
 than one 16-byte load takes.
 """
+import ctypes as C
 import sys
 
 import numpy as np
@@ -51,7 +52,8 @@ def _run(bx, orc, dt, ta, tb, M, N, K, pad, off, seed):
 
 # (M, N, K): one below, at and above the edges of the 32, 64 and 128 row tiles
 # and of the K tiles (32 FP32, 16 FP64, 8 complex), K shorter than the pipeline
-# and longer, grids that pick each shape
+# and longer.  The library takes 32x32 and 64x32 tiles for these; the test of
+# given shapes below runs the others.
 SHAPES = [(1, 1, 1), (2, 3, 5), (31, 33, 7), (32, 32, 32), (33, 31, 65), (63, 65, 129), (64, 64, 64),
           (65, 129, 31), (96, 40, 1000), (129, 127, 48), (700, 600, 40), (1030, 515, 33),
           (1300, 1500, 24)]
@@ -70,7 +72,8 @@ def test_tile_edges_integer_exact(gpu, orc, dt, pad, off):
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
 def test_large_tile_integer_exact(gpu, orc, dt):
-    """a grid that takes the 128 x 64 tile, ragged in both dimensions"""
+    """ragged in both dimensions, on the shape that the library takes for it: 128
+    x 64 in FP64, 64 x 32 in FP32"""
     for ta, tb in (("N", "N"), ("T", "T")):
         M, N, K = 4100, 4036, 100
         say("large tile", np.dtype(dt).name, ta, tb, M, N, K)
@@ -85,3 +88,119 @@ def test_large_tile_integer_exact(gpu, orc, dt):
         assert np.array_equal(dC.download(), (opa.astype(np.float64) @ opb.astype(np.float64)).astype(dt))
         for d in (dA, dB, dC):
             d.free()
+
+
+def _tile_fn(bx):
+    T = bx.test_lib()
+    vp, i64 = C.c_void_p, C.c_int64
+    T.bxtest_gemm_tile.argtypes = [C.c_int] * 8 + [vp, vp, i64, vp, i64, vp, i64, vp, vp, i64]
+    return T.bxtest_gemm_tile
+
+
+def _pair(v):
+    return (C.c_double * 2)(complex(v).real, complex(v).imag)
+
+
+DT = {"S": np.float32, "D": np.float64, "Z": np.complex128}
+# (type, padding, offset) -> shapes: by DMA with both 0, else through registers
+# (a complex operand is misaligned by its base alone: half an element)
+KINDS = [("S", 0, 0, 4), ("S", 1, 0, 3), ("D", 0, 0, 5), ("D", 1, 0, 3), ("Z", 0, 0, 4),
+         ("Z", 0, 8, 3)]
+GIVEN = [(t, pad, off, s) for t, pad, off, n in KINDS for s in range(n)]
+ROWS = [32, 64, 64, 128, 128]
+
+
+def _operand(bx, x, off):
+    """x in HBM `off` bytes past a 16-byte boundary, and its address"""
+    raw = np.concatenate([np.zeros(off, np.uint8), x.ravel(order="F").view(np.uint8),
+                          np.zeros(-(off + x.nbytes) % 8, np.uint8)])
+    d = bx.DeviceArray.from_host(raw.view(np.float64)[:, None])
+    return d, d.ptr + off
+
+
+def _even(n, dt, pad):
+    """n rounded up to a 16-byte multiple of elements, plus pad"""
+    per = max(16 // np.dtype(dt).itemsize, 1)
+    return -(-n // per) * per + pad
+
+
+@pytest.mark.parametrize("t,pad,off,shape", GIVEN)
+def test_given_tile_integer_exact(gpu, t, pad, off, shape):
+    """each compiled shape and movement on products around its tile edges and on
+    a grid of several tile groups, every transposition; NaN in the C that beta =
+    0 must not read"""
+    bx, dt = gpu, DT[t]
+    fn, code = _tile_fn(bx), bx.dtype_code(dt)
+    e, cplx = ROWS[shape], t == "Z"
+    ops = [(a, b) for a in range(3 if cplx else 2) for b in range(3 if cplx else 2)]
+    op = (lambda x: x, lambda x: x.T, lambda x: x.conj().T)
+    rng = np.random.default_rng(shape)
+    for M, N, K in [(e, e, 64), (e - 1, e + 1, 47), (2 * e + 1, e - 1, 9), (5, 3, 131),
+                    (9 * e + 7, 3 * e + 5, 39), (3 * e, 21 * e, 96)]:
+        al, be = (2 - 1j, 1 + 3j) if cplx else (3.0, -2.0)
+        for j, (oa, ob) in enumerate(ops if M * N < 40000 else ops[shape % 2::2]):
+            say("given tile", t, pad, off, shape, M, N, K, oa, ob)
+            b0 = j % 2 == 1
+            m = 4 if t == "S" else 64
+            sa, sb = ((M, K) if oa == 0 else (K, M)), ((K, N) if ob == 0 else (N, K))
+            lda, ldb = _even(sa[0], dt, pad), _even(sb[0], dt, pad)
+            A, B, C0 = (_ints(rng, dt, x, m) for x in ((lda, sa[1]), (ldb, sb[1]), (M + pad, N)))
+            prod = op[oa](A[:sa[0]]) @ op[ob](B[:sb[0]])  # exact in the element type
+            ref = C0.copy(order="F")
+            ref[:M] = al * prod + (0 if b0 else be * C0[:M])
+            if b0:
+                C0[:M] = np.nan
+            (dA, pA), (dB, pB) = _operand(bx, A, off), _operand(bx, B, off)
+            dC = bx.DeviceArray.from_host(C0)
+            rc = fn(code, shape, 0, oa, ob, M, N, K, _pair(al), pA, lda, pB, ldb, None, 0,
+                    _pair(0 if b0 else be), dC.ptr, M + pad)
+            assert rc == 0
+            bx.synchronize()
+            out = dC.download()
+            for d in (dA, dB, dC):
+                d.free()
+            assert np.array_equal(out, ref), (t, pad, off, shape, M, N, K, oa, ob)
+
+
+@pytest.mark.parametrize("t,pad,off,shape", GIVEN)
+def test_given_tile_triangles_integer_exact(gpu, t, pad, off, shape):
+    """rank-k (and rank-2k) triangles on each compiled shape and movement: the
+    stored triangle exact, the diagonal of a Hermitian update real, the other
+    triangle untouched"""
+    bx, dt = gpu, DT[t]
+    fn, code = _tile_fn(bx), bx.dtype_code(dt)
+    e, cplx = ROWS[shape], t == "Z"
+    rng = np.random.default_rng(shape)
+    m = 4 if t == "S" else 64
+    for N, K in [(1, 20), (e - 1, 33), (e + 1, 8), (5 * e + 3, 40), (11 * e, 17)]:
+        for j, (tri, opa) in enumerate([(1, 0), (2, 1), (2, 0), (1, 1)]):
+            herm = cplx and j % 2 == 0
+            two = j >= 2  # a second K segment: B op(A)^T
+            say("given triangle", t, pad, off, shape, N, K, tri, opa, herm, two)
+            oa = opa * (2 if herm else 1)
+            ob = 0 if opa else (2 if herm else 1)
+            sh = (K, N) if opa else (N, K)
+            ld = _even(sh[0], dt, pad)
+            A, B, C0 = (_ints(rng, dt, x, m) for x in ((ld, sh[1]), (ld, sh[1]), (N + pad, N)))
+            X, Y = ((x[:sh[0]].T if opa else x[:sh[0]]) for x in (A, B))  # op(A) = X, or conj(X)
+            tr = (lambda x: x.conj().T) if herm else (lambda x: x.T)
+            if opa and herm:
+                X, Y = X.conj(), Y.conj()
+            al = 2.0 if herm or not cplx else 2 - 1j
+            be = -1.0 if herm or not cplx else 1 + 3j
+            full = al * (X @ tr(Y) + Y @ tr(X) if two else X @ tr(X)) + be * C0[:N]
+            if herm:
+                full[np.diag_indices(N)] = full[np.diag_indices(N)].real
+            keep = np.tril(np.ones((N, N), bool)) if tri == 1 else np.triu(np.ones((N, N), bool))
+            ref = C0.copy(order="F")
+            ref[:N][keep] = full[keep]
+            (dA, pA), (dB, pB) = _operand(bx, A, off), _operand(bx, B, off)
+            dC = bx.DeviceArray.from_host(C0)
+            rc = fn(code, shape, tri | (4 if herm else 0), oa, ob, N, N, K, _pair(al), pA, ld,
+                    pB if two else pA, ld, pB if two else None, ld, _pair(be), dC.ptr, N + pad)
+            assert rc == 0
+            bx.synchronize()
+            out = dC.download()
+            for d in (dA, dB, dC):
+                d.free()
+            assert np.array_equal(out, ref), (t, pad, off, shape, N, K, tri, opa, herm, two)

@@ -4,13 +4,19 @@ the library's own rules, without a GPU.  Shapes of a single product: 0 32x32,
 128x128, 1 128x64, 2 64x64, 3 32x32."""
 import ctypes as C
 
+import numpy as np
 import pytest
+
+DIMS = [(32, 32), (64, 32), (64, 64), (128, 64), (128, 128)]
+LOWER, UPPER = 1, 2
 
 
 @pytest.fixture(scope="module")
 def L(bx):
     T = bx.test_lib()
     T.bxtest_tile_shape.argtypes = [C.c_int] * 5 + [C.c_int64]
+    T.bxtest_tile_walk.argtypes = [C.c_int] * 4 + [C.c_void_p, C.c_int64]
+    T.bxtest_tile_walk.restype = C.c_int64
     return T
 
 
@@ -67,3 +73,76 @@ def test_complex_rounds_of_the_tile_runtime(bx, L):
     L.bxtest_round_tile(bx.Z, 8192, 0, 0, 8192, 8192, 8192, C.byref(shape), C.byref(form),
                         C.byref(grid))
     assert (shape.value, grid.value) == (1, -1)
+
+
+# every shape that a plain or rank-k launch can take, with a product and a
+# triangle that takes it: (type, by DMA, shape, (M, N, K), (N, K))
+REACHED = [
+    ("S", 1, 0, (300, 300, 300), (300, 300)), ("S", 1, 1, (9080, 345, 3), (2497, 9)),
+    ("S", 1, 2, (36433, 2809, 3), (17059, 8)), ("S", 1, 3, (64847, 51209, 18093), (50381, 51477)),
+    ("S", 0, 0, (134, 20, 65224), (100, 42057)), ("S", 0, 1, (54692, 92, 8), (3837, 642)),
+    ("S", 0, 2, (49665, 4309, 3), (19331, 36)),
+    ("D", 1, 0, (2960, 1, 4151), (356, 5432)), ("D", 1, 1, (13508, 15, 262), (2668, 1)),
+    ("D", 1, 2, (4555, 413, 978), (4099, 565)), ("D", 1, 3, (627, 16269, 665), (37183, 3)),
+    ("D", 1, 4, (5304, 701, 14400), (63076, 53963)),
+    ("D", 0, 0, (200, 4591, 941), (168, 4000)), ("D", 0, 1, (3784, 79, 260), (3061, 72)),
+    ("D", 0, 2, (806, 3520, 777), (8886, 189)),
+    ("Z", 1, 0, (211, 3000, 77), (200, 745)), ("Z", 1, 1, (10395, 25, 2677), (3601, 15)),
+    ("Z", 1, 2, (13363, 36, 14823), (2651, 2011)), ("Z", 1, 3, (16384, 16384, 4096), (36851, 3)),
+    ("Z", 0, 0, (725, 36, 67), (212, 2000)), ("Z", 0, 1, (11216, 31, 13726), (707, 11637)),
+    ("Z", 0, 2, (2490, 2823, 259), (8645, 1)),
+]
+
+
+def test_shapes_taken_per_type(bx, L):
+    """the shapes compiled for plain launches are those that the costs can
+    pick: each is taken by some product and some triangle, and no other is"""
+    code = {"S": bx.S, "D": bx.D, "Z": bx.Z}
+    have = {"S1": 4, "S0": 3, "D1": 5, "D0": 3, "Z1": 4, "Z0": 3}
+    assert {k: len({r[2] for r in REACHED if f"{r[0]}{r[1]}" == k}) for k in have} == have
+    for t, dma, s, (m, n, k), (tn, tk) in REACHED:
+        assert L.bxtest_tile_shape(code[t], dma, 0, m, n, k) == s, (t, dma, s)
+        assert L.bxtest_tile_shape(code[t], dma, LOWER, tn, tn, tk) == s, (t, dma, s)
+    rng = np.random.default_rng(1)
+    for m, n, k in np.exp(rng.uniform(0, np.log(65536), (20000, 3))).astype(int) + 1:
+        for t in code:
+            for dma in (0, 1):
+                for tri in (0, LOWER):
+                    s = L.bxtest_tile_shape(code[t], dma, tri, m, m if tri else n, k)
+                    assert s < have[f"{t}{dma}"], (t, dma, tri, m, n, k, s)
+
+
+def _walk(L, shape, tri, m, n, cap=400000):
+    buf = np.empty((cap, 2), np.int32)
+    k = L.bxtest_tile_walk(shape, tri, m, n, buf.ctypes.data, cap)
+    assert k >= 0
+    return buf[:k]
+
+
+@pytest.mark.parametrize("shape", range(5))
+def test_triangle_walk_takes_each_tile_once(bx, L, shape):
+    """every tile with an element on the stored triangle, once; the rest of the
+    grid are tiles of the matrix beside the diagonal, each once too"""
+    bm, bn = DIMS[shape]
+    rng = np.random.default_rng(shape)
+    for n in [1, 2, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 300, 1000, 1024, 2100,
+              4000] + list(rng.integers(1, 5000, 12)):
+        tm, tn = -(-n // bm), -(-n // bn)
+        for tri in (LOWER, UPPER):
+            got = _walk(L, shape, tri, n, n)
+            seen = np.zeros((tm, tn), int)
+            np.add.at(seen, (got[:, 0], got[:, 1]), 1)  # IndexError outside the matrix
+            assert got.min() >= 0 and seen.max() == 1, (n, tri)
+            r0, c0 = np.arange(tm) * bm, np.arange(tn) * bn
+            r1, c1 = np.minimum(r0 + bm, n) - 1, np.minimum(c0 + bn, n) - 1
+            need = (r1[:, None] >= c0) if tri == LOWER else (r0[:, None] <= c1)
+            assert np.all(seen[need] == 1), (n, tri)
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (500, 130), (129, 5000), (4097, 1000), (640, 640),
+                                 (3000, 9000), (16384, 8192)])
+def test_striped_walk_takes_each_tile_once(bx, L, m, n):
+    got = _walk(L, 4, 0, m, n)
+    tm, tn = -(-m // 128), -(-n // 128)
+    assert len(got) == tm * tn
+    assert np.array_equal(np.unique(got[:, 0] * tn + got[:, 1]), np.arange(tm * tn))
