@@ -156,7 +156,7 @@ BX_EXPORT int blasx_tune_table_add(int dtype, int M, int N, int K, int T)
 
 /* ---- block tile shapes of the grouped launches ------------------------------
  * A grouped launch runs each real problem on 128 x 128, 128 x 64 or 64 x 64
- * block tiles (BXH_SHAPE_*); complex problems keep 128 x 64.  Smaller tiles
+ * block tiles (BXH_SHAPE_*; complex problems: grouped.c).  Smaller tiles
  * give a launch with few tiles more blocks to spread over the CUs, at a
  * lower rate per tile.  The table holds measured launch times per shape for
  * workloads of equal problems (tune_grouped.inc, written by

@@ -6,8 +6,9 @@
  *
  * Descriptors are turned into a device-resident table of bxh_problem_t
  * (one block-tile range each) and bxh_seg_t (one K segment each) consumed
- * by the grouped kernel; blocks walk the table with a grid stride, so a
- * 64^3 request and an 8192^3 request share one launch without a tail.
+ * by the grouped kernel: a block finds its problem by its tile number (a graph
+ * replay's blocks walk the tiles with a grid stride), the problems of the longest
+ * K first, so a 64^3 request and an 8192^3 request share a launch.
  */
 #include <pthread.h>
 #include <stdlib.h>

@@ -206,10 +206,12 @@ typedef struct blasx_gemm_desc {
 
 int blasx_gemm_grouped_device(const blasx_gemm_desc_t *descs, int n, void *stream);
 
-/* Block tile shape of a real problem in a grouped launch (or a server
- * batch): 0 = 128 x 128, 1 = 128 x 64, 2 = 64 x 64 (which a launch with too
- * few tiles cuts to 32 x 32).  Complex problems, and operands without
- * 16-byte alignment, take the nearest shape that they have.  No counterpart in the reference (its tile sizes are compile-time
+/* Block tile shape of a real problem in a grouped launch: 0 = 128 x 128, 1 =
+ * 128 x 64, 2 = 64 x 64 (which a launch with too few tiles cuts to 32 x 32).
+ * Operands without 16-byte alignment, and every problem of a server batch
+ * (one captured launch), run on the last two whatever is asked; complex
+ * problems take 128 x 64 or smaller by a rule of their own.  No counterpart in
+ * the reference (its tile sizes are compile-time
  * constants, include/blasx.h:5-7).  The shape is picked per problem from a
  * table of launch times measured on an MI355X (built in, written by
  * python -m blasx_amd.tune --grouped; entries added at run time carry a
