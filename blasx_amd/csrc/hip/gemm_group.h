@@ -125,6 +125,8 @@ int launch_group(const bxh_problem_t *probs, int nprob, const bxh_seg_t *segs, i
         hipLaunchKernelGGL(k_group_big<E>, dim3(total), dim3(NT), 0, st, probs, nprob, segs);
     } else {
         if (grid <= 0 || (!counts && grid > total)) grid = total;
+        // a grid's threads fit 32 bits: beyond, blocks take several tiles
+        if (grid >= (1 << 24)) grid = (1 << 24) - 1;
         hipLaunchKernelGGL(k_group<E>, dim3(grid), dim3(NT), 0, st, probs, nprob, segs, total, counts);
     }
     return bx_launch_status("grouped gemm launch");

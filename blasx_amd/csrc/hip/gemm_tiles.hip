@@ -39,6 +39,12 @@ __global__ __launch_bounds__(NT, OCC) void k_tile(bxh_problem_t P, bxh_seg_t S, 
     tile_block<E, MAJA, MAJB, CJA, CJB, WTM, WTN, NS, DMA>(P, nullptr, S, S1, tm, tn, smem);
 }
 
+// A launch's threads fit 32 bits along a dimension, and a tile's rows an int.
+// Skinny products of hundreds of millions of columns would have more tiles
+// of 32x32 (or 64 rows) than that.
+constexpr int64_t MOST_TILES = ((int64_t)1 << 32) / NT - 1;
+constexpr int MOST_ROWS = INT32_MAX - 127;
+
 template <int BM, int BN> int64_t grid_tiles(int tri, int m, int n)
 {
     const int tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
@@ -95,15 +101,19 @@ void launch_shape(bxh_problem_t P, const bxh_seg_t *S, hipStream_t st)
 namespace {
 
 // the shape that runs one product fastest (tilecost.h; all tiles alike, so
-// the busiest CU has the rounded-up share)
-int best_shape(int dtype, bool dma, int tri, int m, int n, int64_t k)
+// the busiest CU has the rounded-up share) in at most `most` tiles; the
+// largest tile where none does
+int best_shape(int dtype, bool dma, int tri, int m, int n, int64_t k, int64_t most)
 {
     int best = BXC_32x32;
     double bt = 1e300;
     for (int s = BXC_32x32; s < BXC_SHAPES; ++s) {
         const bx_cost_t &c = dma ? BX_COST_DMA[dtype][s] : BX_COST_REG[dtype][s];
         if (c.a <= 0) continue;
-        const double t = c.l + (double)((shape_tiles(s, tri, m, n) + 255) / 256) * bx_cost_tile(&c, k);
+        const int64_t tiles = shape_tiles(s, tri, m, n);
+        if (bt == 1e300) best = s;
+        if (tiles > most) continue;
+        const double t = c.l + (double)((tiles + 255) / 256) * bx_cost_tile(&c, k);
         if (t < bt) {
             bt = t;
             best = s;
@@ -144,10 +154,12 @@ bool launch_tile(int s, const bxh_problem_t &P, const bxh_seg_t *S, hipStream_t 
 
 extern "C" {
 
-int bxh_gemm_tile_as(int dtype, int shape, const bxh_problem_t *P, const bxh_seg_t *S, void *stream)
+int bxh_gemm_tile_most(int dtype, int shape, const bxh_problem_t *P, const bxh_seg_t *S, void *stream,
+                       int64_t most)
 {
     if (dtype < 0 || dtype > 2 || P->nseg < 1 || P->nseg > 2 || (P->tri && P->m != P->n))
         return BLASX_EINVAL;
+    const int big = P->m > P->n ? P->m : P->n;
     bxh_problem_t Q = *P;
     Q.form = BXH_FORM_DMA;
     int64_t k = 0;
@@ -156,14 +168,42 @@ int bxh_gemm_tile_as(int dtype, int shape, const bxh_problem_t *P, const bxh_seg
         Q.form = f > Q.form ? f : Q.form;
         k += S[i].k;
     }
+    int s = shape;
+    if (big <= MOST_ROWS) {
+        if (s < 0) s = best_shape(dtype, Q.form == BXH_FORM_DMA, P->tri, P->m, P->n, k, most);
+        if (s >= BXC_SHAPES) return BLASX_EINVAL;
+    }
+    if (!P->tri && big > 128 && (big > MOST_ROWS || shape_tiles(s, 0, P->m, P->n) > most)) {
+        // too many tiles for one launch: the longer side in halves
+        const int es = dtype == BLASX_S ? 4 : dtype == BLASX_D ? 8 : 16;
+        const bool rows = P->m == big;
+        const int64_t h = ((int64_t)big / 2 + 127) / 128 * 128;
+        bxh_seg_t S2[2];
+        for (int i = 0; i < P->nseg; ++i) {
+            S2[i] = S[i];
+            if (rows)
+                S2[i].A = (const char *)S[i].A + (P->opa == 0 ? h : h * S[i].lda) * es;
+            else
+                S2[i].B = (const char *)S[i].B + (P->opb == 0 ? h * S[i].ldb : h) * es;
+        }
+        (rows ? Q.m : Q.n) = (int)h;
+        const int rc = bxh_gemm_tile_most(dtype, shape, &Q, S, stream, most);
+        if (rc) return rc;
+        (rows ? Q.m : Q.n) = big - (int)h;
+        Q.C = (char *)P->C + (rows ? h : h * P->ldc) * es;
+        return bxh_gemm_tile_most(dtype, shape, &Q, S2, stream, most);
+    }
     hipStream_t st = (hipStream_t)stream;
-    const int s =
-        shape >= 0 ? shape : best_shape(dtype, Q.form == BXH_FORM_DMA, P->tri, P->m, P->n, k);
     const bool ran = dtype == BLASX_S   ? launch_tile<float>(s, Q, S, st)
                      : dtype == BLASX_D ? launch_tile<double>(s, Q, S, st)
                                         : launch_tile<cplx>(s, Q, S, st);
     if (!ran) return BLASX_EINVAL;
     return bx_launch_status(P->tri ? "rank-k launch" : "gemm launch");
+}
+
+int bxh_gemm_tile_as(int dtype, int shape, const bxh_problem_t *P, const bxh_seg_t *S, void *stream)
+{
+    return bxh_gemm_tile_most(dtype, shape, P, S, stream, MOST_TILES);
 }
 
 int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *stream)
@@ -195,7 +235,7 @@ int bxh_tile_at_host(int shape, int tri, int m, int n, int64_t t, int *tm, int *
 }
 int bxh_tile_shape_host(int dtype, int dma, int tri, int m, int n, int64_t k)
 {
-    return best_shape(dtype, dma != 0, tri, m, n, k);
+    return best_shape(dtype, dma != 0, tri, m, n, k, MOST_TILES);
 }
 
 } // extern "C"

@@ -137,6 +137,9 @@ int bxh_gemm_tile(int dtype, const bxh_problem_t *P, const bxh_seg_t *S, void *s
 /* on the given shape (BXC_*, tilecost.h); BLASX_EINVAL where the type and form
  * of the operands have no such tile */
 int bxh_gemm_tile_as(int dtype, int shape, const bxh_problem_t *P, const bxh_seg_t *S, void *stream);
+/* in launches of at most `most` tiles each (bxh_gemm_tile_as: what a grid holds) */
+int bxh_gemm_tile_most(int dtype, int shape, const bxh_problem_t *P, const bxh_seg_t *S, void *stream,
+                       int64_t most);
 /* grouped launch over a device-resident problem and segment table; all
  * problems share dtype.  grid = 0: one block per tile, every problem's shape
  * BXH_SHAPE_64x64 or BXH_SHAPE_32x32; grid = BXH_GROUP_BIG: one block per

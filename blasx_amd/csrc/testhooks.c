@@ -156,12 +156,12 @@ BX_EXPORT int bxtest_round_tile(int dt, int T, int opa, int opb, int M, int N, i
 }
 
 /* the plain GEMM and rank-k launch on a given block tile shape (BXC_*; -1:
- * the one the library takes); B2 non-NULL: a second K segment, B2 op(A)^T;
- * and the shape the library takes */
-BX_EXPORT int bxtest_gemm_tile(int dt, int shape, int tri, int opa, int opb, int m, int n, int k,
-                               const double *alpha, const void *A, int64_t lda, const void *B,
-                               int64_t ldb, const void *B2, int64_t ldb2, const double *beta,
-                               void *C, int64_t ldc)
+ * the one the library takes), in launches of at most `most` tiles; B2 non-NULL:
+ * a second K segment, B2 op(A)^T; and the shape the library takes */
+BX_EXPORT int bxtest_gemm_tile_most(int dt, int shape, int tri, int opa, int opb, int m, int n, int k,
+                                    const double *alpha, const void *A, int64_t lda, const void *B,
+                                    int64_t ldb, const void *B2, int64_t ldb2, const double *beta,
+                                    void *C, int64_t ldc, int64_t most)
 {
     bxh_problem_t P = {0};
     P.C = C;
@@ -174,7 +174,16 @@ BX_EXPORT int bxtest_gemm_tile(int dt, int shape, int tri, int opa, int opb, int
     P.beta_re = beta[0], P.beta_im = beta[1];
     P.beta_zero = beta[0] == 0.0 && beta[1] == 0.0;
     const bxh_seg_t S[2] = {{A, B, lda, ldb, k}, {B2, A, ldb2, lda, k}};
-    return bxh_gemm_tile_as(dt, shape, &P, S, NULL);
+    return most ? bxh_gemm_tile_most(dt, shape, &P, S, NULL, most)
+                : bxh_gemm_tile_as(dt, shape, &P, S, NULL);
+}
+BX_EXPORT int bxtest_gemm_tile(int dt, int shape, int tri, int opa, int opb, int m, int n, int k,
+                               const double *alpha, const void *A, int64_t lda, const void *B,
+                               int64_t ldb, const void *B2, int64_t ldb2, const double *beta,
+                               void *C, int64_t ldc)
+{
+    return bxtest_gemm_tile_most(dt, shape, tri, opa, opb, m, n, k, alpha, A, lda, B, ldb, B2, ldb2,
+                                 beta, C, ldc, 0);
 }
 int bxh_tile_at_host(int shape, int tri, int m, int n, int64_t t, int *tm, int *tn);
 /* the tiles of every block of a launch into tiles[2 t]; how many (-1: more than cap) */

@@ -204,3 +204,48 @@ def test_given_tile_triangles_integer_exact(gpu, t, pad, off, shape):
             for d in (dA, dB, dC):
                 d.free()
             assert np.array_equal(out, ref), (t, pad, off, shape, N, K, tri, opa, herm, two)
+
+
+@pytest.mark.parametrize("t", ["S", "D", "Z"])
+def test_product_cut_into_launches_integer_exact(gpu, t):
+    """what has more tiles than a launch may hold is cut into several: here at a
+    few tiles, tall, wide and square, every transposition, with padding"""
+    bx, dt = gpu, DT[t]
+    fn, code = _tile_fn(bx), bx.dtype_code(dt)
+    fn = bx.test_lib().bxtest_gemm_tile_most
+    fn.argtypes = bx.test_lib().bxtest_gemm_tile.argtypes + [C.c_int64]
+    cplx = t == "Z"
+    op = (lambda x: x, lambda x: x.T, lambda x: x.conj().T)
+    al, be = (2 - 1j, 1 + 3j) if cplx else (3.0, -2.0)
+    rng = np.random.default_rng(5)
+    for M, N, K, most in [(1000, 3, 20, 4), (5, 1100, 33, 3), (700, 650, 24, 7), (200, 130, 8, 1)]:
+        for oa in range(3 if cplx else 2):
+            for ob in range(3 if cplx else 2):
+                say("cut product", t, M, N, K, most, oa, ob)
+                sa, sb = ((M, K) if oa == 0 else (K, M)), ((K, N) if ob == 0 else (N, K))
+                A, B, C0 = (_ints(rng, dt, (r + 4, c), 4) for r, c in (sa, sb, (M, N)))
+                ref = C0.copy(order="F")
+                ref[:M] = al * (op[oa](A[:sa[0]]) @ op[ob](B[:sb[0]])) + be * C0[:M]
+                dA, dB, dC = (bx.DeviceArray.from_host(x) for x in (A, B, C0))
+                rc = fn(code, -1, 0, oa, ob, M, N, K, _pair(al), dA.ptr, sa[0] + 4, dB.ptr,
+                        sb[0] + 4, None, 0, _pair(be), dC.ptr, M + 4, most)
+                assert rc == 0
+                bx.synchronize()
+                out = dC.download()
+                for d in (dA, dB, dC):
+                    d.free()
+                assert np.array_equal(out, ref), (t, M, N, K, most, oa, ob)
+
+
+def test_skinny_product_of_600_million_columns(gpu):
+    """more columns than a grid of 32-column tiles holds"""
+    bx, n = gpu, 600_000_000
+    A = bx.DeviceArray.from_host(np.full((1, 1), 3, np.float32))
+    B, Cd = bx.DeviceArray(1, n, np.float32), bx.DeviceArray(1, n, np.float32)
+    B.fill_uniform(1, 1)
+    say("skinny", n)
+    bx.device_gemm("N", "N", 1, n, 1, 1.0, A.ptr, 1, B.ptr, 1, 0.0, Cd.ptr, 1, np.float32)
+    bx.synchronize()
+    assert np.array_equal(Cd.download(), np.float32(3) * B.download())
+    for d in (A, B, Cd):
+        d.free()

@@ -146,3 +146,19 @@ def test_striped_walk_takes_each_tile_once(bx, L, m, n):
     tm, tn = -(-m // 128), -(-n // 128)
     assert len(got) == tm * tn
     assert np.array_equal(np.unique(got[:, 0] * tn + got[:, 1]), np.arange(tm * tn))
+
+
+def test_tiles_of_a_launch_fit_its_grid(bx, L):
+    """a launch of 256 threads a tile takes fewer than 2^24 tiles: long skinny
+    products (all within a GPU's memory) take a larger tile where a small one
+    would have more; only beyond the largest tile is a product cut"""
+    code = {"S": bx.S, "D": bx.D, "Z": bx.Z}
+    for t, dma, m, n, k in [("D", 1, 131, 162670080, 85), ("D", 1, 1, 600_000_000, 4),
+                            ("S", 1, 67, 1044287977, 1), ("S", 1, 600_000_000, 1, 1),
+                            ("S", 0, 64, 900_000_000, 2), ("D", 0, 65, 522693628, 2),
+                            ("Z", 1, 1_000_000_000, 3, 1), ("Z", 0, 1_000_000_000, 3, 1)]:
+        bm, bn = DIMS[L.bxtest_tile_shape(code[t], dma, 0, m, n, k)]
+        assert -(-m // bm) * -(-n // bn) < 2**24, (t, dma, m, n, k)
+    for t in code:
+        bm, bn = DIMS[L.bxtest_tile_shape(code[t], 1, LOWER, 265264, 265264, 680)]
+        assert -(-265264 // bm) * -(-265264 // bn) / 2 < 2**24
