@@ -1279,7 +1279,7 @@ def main():
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py: this build targets one GPU; --gpus {args.gpus} is not supported "
-              "(the multi-GPU design is described in DESIGN.md, not built)", file=sys.stderr)
+              "(no multi-GPU path is built)", file=sys.stderr)
         sys.exit(2)
 
     import blasx_amd as bx
